@@ -80,11 +80,12 @@ hip_moe_layer *hip_moe_upload(const float *gate_inp,
  * a Q4_K_M GGUF keeps gate/up in Q4_K and down in Q6_K or Q4_K.  Q8_0/Q4_0
  * need gate_type == down_type (then this is hip_moe_upload).  K-quant
  * experts (gate/up and down each HIP_MOE_Q4_K or HIP_MOE_Q6_K; E a multiple
- * of 256 up to 8192, EI up to 16384) stay as the tensors' rows and take one
- * path for every T: routing, then per (token, slot) the Q8_K integer
+ * of 256 up to 8192, EI up to 16384) stay as the tensors' rows and take the
+ * same arithmetic for every T: routing, then per (token, slot) the Q8_K integer
  * gate/up dots of the reference's -DQ8_DOT build, SwiGLU, and the fp32 down
  * dot in the reference's own order (fused_ffn_silu, nn.c:449-539), then the
- * combine; outputs, ids and weights equal the reference's bit for bit.
+ * combine (many tokens: the pairs sorted by expert, the same dots on the
+ * matrix cores); outputs, ids and weights equal the reference's bit for bit.
  */
 hip_moe_layer *hip_moe_upload_typed(const float *gate_inp,
                                     const void *const *gate_e,

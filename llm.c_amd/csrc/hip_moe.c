@@ -62,6 +62,8 @@ struct hip_moe_layer {
 	int *d_tile_e;      /* grouped path: expert of each m-tile, -1 = unused */
 	void *d_h16;        /* grouped path: f16 h in sorted row order */
 	void *d_xh;         /* grouped path: tokens rounded to f16 [T][E] */
+	void *d_rec;        /* K-quant experts, many tokens: their Q8_K records */
+	float *d_hs;        /* and h in sorted row order */
 
 	/* staging for the host-pointer entry point */
 	size_t cap_io;
@@ -218,6 +220,8 @@ void hip_moe_free(hip_moe_layer *L)
 	hipFree(L->d_tile_e);
 	hipFree(L->d_h16);
 	hipFree(L->d_xh);
+	hipFree(L->d_rec);
+	hipFree(L->d_hs);
 	hipFree(L->d_x);
 	hipFree(L->d_out);
 	hipFree(L->d_bias);
@@ -367,6 +371,31 @@ size_t hip_moe_weight_bytes(const hip_moe_layer *L)
 	return L ? L->weight_bytes : 0;
 }
 
+/* 32-row tiles a sort of P pairs can use, and whether the grouped K-quant
+ * products (kq_grouped.hip) take a call of T tokens.  The other kernels read
+ * an expert's weights once per pair, these once per expert and 32 pairs but
+ * in five more launches: taken once the pairs past one per expert would
+ * re-read KQ_GROUPED_BYTES.  Measured either side of it (Q4_K gate/up, Q6_K
+ * down; per pair / grouped): 2048 x 1024, 64 experts top-8, T=8 130 / 117
+ * us, T=12 164 / 124; 4096 x 14336, 8 top-2, T=4 317 / 356, T=8 610 / 389;
+ * 1024 x 512, 64 top-8, T=9 47 / 54, T=12 56 / 56, T=16 69 / 57; 2048 x
+ * 1024, 8 top-2, T=8 48 / 58, T=9 57 / 58, T=16 85 / 58 */
+#define KQ_GROUPED_BYTES ((size_t)40 << 20)
+static size_t kq_tiles(const hip_moe_layer *L, size_t P)
+{
+	const size_t r = (size_t)moe_kq_tile_rows();
+	return (P + r - 1) / r + (L->NE < P ? L->NE : P);
+}
+
+static int kq_grouped_fits(const hip_moe_layer *L, size_t T)
+{
+	const size_t P = T * L->topk;
+	return P > L->NE &&
+	       (P - L->NE) * (2 * L->gu_stride + L->down_stride) >= KQ_GROUPED_BYTES &&
+	       kq_tiles(L, P) <= (size_t)moe_prefill_tile_cap() &&
+	       moe_kq_rec_bytes(T, L->E) <= 0xffffffffull;
+}
+
 /*
  * Scratch for calls of up to T tokens.  Growing it frees the old buffers,
  * which a HIP graph captured earlier would still name, so growth is refused
@@ -398,8 +427,12 @@ static int ensure_scratch(hip_moe_layer *L, size_t T, hipStream_t s)
 	hipFree(L->d_tile_e);
 	hipFree(L->d_h16);
 	hipFree(L->d_xh);
+	hipFree(L->d_rec);
+	hipFree(L->d_hs);
 	L->d_part = NULL;
 	L->d_xh = NULL;
+	L->d_rec = NULL;
+	L->d_hs = NULL;
 	L->d_rows = NULL;
 	L->d_tile_e = NULL;
 	L->d_h16 = NULL;
@@ -449,6 +482,17 @@ static int ensure_scratch(hip_moe_layer *L, size_t T, hipStream_t s)
 		       "hipMalloc(tiles)");
 		HIPCHK(hipMalloc(&L->d_h16, rows * L->EI * 2), "hipMalloc(h16)");
 		HIPCHK(hipMalloc(&L->d_xh, T * L->E * 2), "hipMalloc(xh)");
+	}
+	if (L->kq && kq_grouped_fits(L, T)) {
+		const size_t tiles = kq_tiles(L, P);
+		HIPCHK(hipMalloc((void **)&L->d_rows, tiles * moe_kq_tile_rows() * sizeof(int)),
+		       "hipMalloc(rows)");
+		HIPCHK(hipMalloc((void **)&L->d_tile_e, (tiles + 1) * sizeof(int)),
+		       "hipMalloc(tiles)");
+		HIPCHK(hipMalloc((void **)&L->d_hs,
+				 tiles * moe_kq_tile_rows() * L->EI * sizeof(float)),
+		       "hipMalloc(sorted h)");
+		HIPCHK(hipMalloc(&L->d_rec, moe_kq_rec_bytes(T, L->E)), "hipMalloc(records)");
 	}
 	L->cap_T = T;
 	L->scratch_gen++;
@@ -793,6 +837,22 @@ int hip_moe_ffn_dev(hip_moe_layer *L, const float *d_x, float *d_out, size_t T,
 	if (!path) {
 		set_err("ffn: the requested path does not apply to this layer and T=%zu", T);
 		return 0;
+	}
+	if (L->kq && L->path == HIP_MOE_PATH_AUTO && L->d_rec && kq_grouped_fits(L, T)) {
+		const int tiles = (int)kq_tiles(L, (size_t)P);
+		if (!route(L, d_x, T, d_router_bias, L->d_logits, NULL, ids, w, NULL, s))
+			return 0;
+		LCHK(moe_launch_kq_rec(d_x, (int)T, (int)L->E, L->d_rec, s), "Q8_K records");
+		LCHK(moe_launch_sort32(ids, P, (int)L->NE, tiles, L->d_rows, L->d_tile_e, s),
+		     "sort by expert");
+		LCHK(moe_launch_kq_grouped(L->wtype, L->dtype, L->d_gate, L->d_up, L->d_down,
+					   L->gu_stride, L->down_stride, L->d_rows, L->d_tile_e,
+					   tiles, L->d_rec, L->d_hs, L->d_ypart, (int)T,
+					   (int)L->topk, (int)L->E, (int)L->EI, s),
+		     "grouped K-quant products");
+		LCHK(moe_launch_combine(L->d_ypart, w, d_out, (int)T, (int)L->topk, (int)L->E, 1, s),
+		     "combine");
+		return 1;
 	}
 	if (path == HIP_MOE_PATH_DECODE && L->kq) {
 		LCHK(moe_launch_kq_route_gateup(L->wtype, d_x, L->d_router, d_router_bias, L->d_gate,

@@ -127,6 +127,20 @@ int moe_kq_down_combine_ok(size_t T, size_t K, size_t E, size_t EI);
 int moe_launch_kq_down_combine(int dt, const uint8_t *down, size_t dn_stride,
                                const uint32_t *ids, const float *w, const float *h, float *out,
                                int T, int K, int E, int EI, void *stream);
+/* Many tokens on K-quant experts (kq_grouped.hip), the same bits: the
+ * tokens' Q8_K records (moe_kq_rec_bytes, once per call), the pairs sorted
+ * by expert into tiles of moe_kq_tile_rows() rows (moe_launch_sort32, at
+ * most Tmax tiles, Tmax + 1 ints of tile_e), then gate/up into h [Tmax *
+ * rows][EI] in sorted row order and down into y [P][E]. */
+size_t moe_kq_rec_bytes(size_t T, size_t K);
+int moe_kq_tile_rows(void);
+int moe_launch_kq_rec(const float *x, int T, int K, void *rec, void *stream);
+int moe_launch_sort32(const uint32_t *ids, int P, int NE, int Tmax, int *rows, int *tile_e,
+                      void *stream);
+int moe_launch_kq_grouped(int gt, int dt, const uint8_t *gate, const uint8_t *up,
+                          const uint8_t *down, size_t gu_stride, size_t dn_stride,
+                          const int *rows, const int *tile_e, int Tmax, const void *rec,
+                          float *h, float *y, int T, int topk, int E, int EI, void *stream);
 /* quantize_row_q8 of T rows of K values: d[T][K/256], qs[T][K], bsums[T][K/256][16] */
 int moe_launch_q8k_quantize(const float *x, int T, int K, float *d, int8_t *qs,
                             int16_t *bsums, void *stream);

@@ -1057,6 +1057,18 @@ extern "C" int moe_prefill_tile_cap(void)
 	return SORT_MAX_TILES;
 }
 
+/* the sort alone, into 32-row tiles (the K-quant experts' products) */
+extern "C" int moe_launch_sort32(const uint32_t *ids, int P, int NE, int Tmax, int *rows,
+				 int *tile_e, void *stream)
+{
+	if (P < 1 || NE < 1 || NE > MOE_MAX_NE || Tmax > SORT_MAX_TILES ||
+	    (size_t)Tmax < pf_tiles((size_t)P, (size_t)NE, 32))
+		return (int)hipErrorInvalidValue;
+	hipLaunchKernelGGL(k_moe_sort<32>, dim3(1), dim3(SORT_THREADS), 0, (hipStream_t)stream, ids, P,
+			   NE, Tmax, rows, tile_e);
+	return (int)hipGetLastError();
+}
+
 extern "C" int moe_launch_prefill(int wtype, const void *xh_, const uint8_t *gate,
 				  const uint8_t *up, const uint8_t *down, size_t gu_stride,
 				  size_t dn_stride, const uint32_t *ids, int *rows, int *tile_e,

@@ -1,0 +1,51 @@
+"""The grouped products of K-quant experts (more pairs than experts) at the
+edges of their tiles: bit for bit the oracle's moe_ffn, and the per-pair
+products' (the forced GEMV path)."""
+import numpy as np
+import pytest
+
+import hipmoe
+import oracle
+from common import SEED, bits
+
+pytestmark = pytest.mark.gpu
+
+Q4K, Q6K = hipmoe.Q4_K, hipmoe.Q6_K
+# types, E, EI, NE, topk, renorm, token counts: one super-block a row; every
+# token on every expert (tiles of 32, 32 + 1, 32 + 16 and 32 + 17 rows);
+# ragged d_ff; tiles of a few rows each; the OLMoE shape
+CASES = {
+    "one_block": (Q4K | Q6K << 8, 256, 256, 4, 1, 0, (340,)),
+    "all_experts": (Q6K, 768, 256, 3, 3, 1, (32, 33, 48, 49)),
+    "ragged_dff": (Q6K | Q4K << 8, 512, 768, 8, 2, 1, (29, 70)),
+    "q4k_down": (Q4K, 1024, 512, 16, 4, 0, (17, 130)),
+    "olmoe": (Q4K | Q6K << 8, 2048, 1024, 64, 8, 0, (10,)),
+}
+REREAD = 40 << 20  # bytes the pairs past one per expert re-read where the path starts
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_gpu_kq_grouped_tiles_vs_oracle(name):
+    wt, E, EI, NE, K, renorm, Ts = CASES[name]
+    lw = hipmoe.synth_layer(SEED, 11, wt, E, EI, NE, 0.02, None)
+    gt, dt = hipmoe.wtypes(wt)
+    expert = 2 * EI * hipmoe.row_bytes(gt, E) + E * hipmoe.row_bytes(dt, EI)
+    M = hipmoe.MoeLayer.from_synth(lw, K, bool(renorm))
+    try:
+        for T in Ts:
+            assert (T * K - NE) * expert >= REREAD
+            x = hipmoe.synth_input(SEED, 0x9600 + T, T, E)
+            x[T // 2] = 0.0  # an all-zero token: every Q8_K scale 0
+            x[0, :256] *= 1e6
+            M.set_path(hipmoe.PATH_AUTO)
+            out, ids, w = M.ffn(x)
+            M.set_path(hipmoe.PATH_GEMV)
+            out_p, ids_p, w_p = M.ffn(x)
+            oout, oids, ow, _, _ = oracle.moe_ffn(x, lw, K, bool(renorm), None)
+            print(f"kq grouped {name} T={T}: {int(np.sum(bits(out) != bits(oout)))} of "
+                  f"{out.size} outputs differ", flush=True)
+            assert np.array_equal(ids, oids) and np.array_equal(bits(w), bits(ow))
+            assert np.array_equal(bits(out), bits(oout))
+            assert np.array_equal(bits(out), bits(out_p)) and np.array_equal(ids, ids_p)
+    finally:
+        M.free()
