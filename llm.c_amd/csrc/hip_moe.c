@@ -1164,7 +1164,11 @@ int hip_moe_qmat_mul_dev(const hip_moe_qmat *W, const float *d_x, size_t T,
 	if (!check_add(W, T, d_add, add_len))
 		return 0;
 	void *s = stream ? stream : (void *)W->stream;
-	if (is_kquant(W->wtype)) {
+	if (is_kquant(W->wtype) && moe_kq_dense_better(W->wtype, W->N, T)) {
+		LCHK(moe_launch_kq_dense(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
+					 add_len == T * W->N, d_out, s),
+		     "kq_dense");
+	} else if (is_kquant(W->wtype)) {
 		LCHK(moe_launch_kq_gemv(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 					add_len == T * W->N, d_out, T == 1 ? W->grid1 : W->grid, s),
 		     "kq_gemv");

@@ -8,11 +8,11 @@
  *   k_kq_rec      every token's Q8_K blocks (quantize_row_q8, quant.c:
  *                 627-654) as matrix-core operands: f16 quants, f16 sums
  *                 of 16 (one record per 256 values), and the scales
- *   k_kq_mm       MOE: per (32-row tile of one expert's pairs, 128 h
- *                 columns) gate, up and h = silu(g) * u in sorted row
- *                 order; else out = add + the dense product
+ *   k_kq_mm       per (32-row tile of one expert's pairs, 128 h columns)
+ *                 gate, up and h = silu(g) * u in sorted row order
  *   k_kq_down_mm  y[pair][i] = dot_f32_quant(h[pair], down row i) per
  *                 (32-row tile, 64 output columns)
+ *   k_kq_dense    out = add + x . W^T per (32 tokens, 128 columns)
  *
  * Why these stay exact.  dot_q4_K_q8_K / dot_q6_K_q8_K (quant_avx2.h:8-209)
  * are exact integer sums per super-block of 256, then a sequential chain of
@@ -175,14 +175,18 @@ template <> struct kmw<5> {
  * sh sums (Q6_K).
  */
 #define KM_LROW (KM_ROWS * 16) /* LDS bytes of one chunk index: the 32 rows */
+/* the same where the kernel quantizes the rows itself: four chunks' stores of
+ * 8 rows then start 16 banks apart (two lanes a bank, the least 512 bytes take) */
+#define KM_LROW_Q (KM_LROW + 64)
 
-__device__ static inline half8_t km_a(const uint8_t *sa, int chunk, int m)
+template <int LR> __device__ static inline half8_t km_a(const uint8_t *sa, int chunk, int m)
 {
-	return *(const half8_t *)(sa + chunk * KM_LROW + m * 16);
+	return *(const half8_t *)(sa + chunk * LR + m * 16);
 }
 
 /* the minima's part: acc_m = fma(-yd * dmin, msum, acc_m) for a lane's 16
  * rows (row 8 q + 4 h + i: yd points at the scales of rows 4 h ..) */
+template <int LR>
 __device__ static inline void km_mins(const kmw<3> &w, const uint8_t *sa, int m, int h,
 				      const floatx4 *yd, floatx16 &accm)
 {
@@ -197,18 +201,20 @@ __device__ static inline void km_mins(const kmw<3> &w, const uint8_t *sa, int m,
 	for (int k = 0; k < 4; k++)
 		mo[2 * k] = mo[2 * k + 1] = (_Float16)(float)((mw >> (8 * k)) & 0xff);
 	const floatx16 M =
-		__builtin_amdgcn_mfma_f32_32x32x16_f16(km_a(sa, 32 + h, m), mo, z, 0, 0, 0);
+		__builtin_amdgcn_mfma_f32_32x32x16_f16(km_a<LR>(sa, 32 + h, m), mo, z, 0, 0, 0);
 	const float dm = f16_bits_to_f32(w.hd.x >> 16);
 #pragma unroll
 	for (int j = 0; j < 16; j++)
 		accm[j] = __builtin_fmaf(-yd[2 * (j / 4)][j % 4] * dm, M[j], accm[j]);
 }
 
+template <int LR>
 __device__ static inline void km_mins(const kmw<5> &, const uint8_t *, int, int, const floatx4 *,
 				      floatx16 &)
 {
 }
 
+template <int LR>
 __device__ static inline void km_sums(const kmw<3> &w, const uint8_t *sa, int m, int h,
 				      floatx16 &S1, floatx16 &S2)
 {
@@ -231,8 +237,8 @@ __device__ static inline void km_sums(const kmw<3> &w, const uint8_t *sa, int m,
 			const u32 x = w.dw(j, 2 * u), y = w.dw(j, 2 * u + 1);
 			const half8_t lo = km_op(x, y, 0x000f000fu, a2, ao2);
 			const half8_t hi = km_op(x, y, 0x00f000f0u, b2, bo2);
-			const half8_t al = km_a(sa, ((4 * j + u) * 2) + h, m);
-			const half8_t ah = km_a(sa, ((4 * j + 2 + u) * 2) + h, m);
+			const half8_t al = km_a<LR>(sa, ((4 * j + u) * 2) + h, m);
+			const half8_t ah = km_a<LR>(sa, ((4 * j + 2 + u) * 2) + h, m);
 			floatx16 &S = j < 2 ? S1 : S2;
 			S = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, lo, S, 0, 0, 0);
 			S = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, hi, S, 0, 0, 0);
@@ -242,6 +248,7 @@ __device__ static inline void km_sums(const kmw<3> &w, const uint8_t *sa, int m,
 	}
 }
 
+template <int LR>
 __device__ static inline void km_sums(const kmw<5> &w, const uint8_t *sa, int m, int h,
 				      floatx16 &S1, floatx16 &S2)
 {
@@ -266,7 +273,7 @@ __device__ static inline void km_sums(const kmw<5> &w, const uint8_t *sa, int m,
 					const u32 lo = g < 2 ? q & 0x0f0f0f0fu : (q >> 4) & 0x0f0f0f0fu;
 					v[k] = lo | (((w.qh[c][2 * u + k] >> (2 * g)) & 0x03030303u) << 4);
 				}
-				const half8_t a = km_a(sa, ((2 * i + u) * 2) + h, m);
+				const half8_t a = km_a<LR>(sa, ((2 * i + u) * 2) + h, m);
 				S1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(
 					a, km_op(v[0], v[1], 0x00ff00ffu, sl2, slo2), S1, 0, 0, 0);
 				S2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(
@@ -297,7 +304,7 @@ __device__ static inline void km_step(const kmw<5> &w, const floatx16 &S1, const
 }
 
 /* ------------------------------------------------------------------ */
-/* gate/up of grouped pairs, and the dense product                      */
+/* gate/up of grouped pairs                                              */
 /* ------------------------------------------------------------------ */
 
 /* workgroup id -> item: the XCDs are dealt workgroups round-robin, so class
@@ -312,8 +319,7 @@ __device__ static inline int km_item(int id, int items)
 
 /*
  * A workgroup of NW waves takes a tile of 32 rows and NW * 32 columns: wave
- * w columns 32 w .. 32 w + 31 of gate and of up (MOE), or of the dense
- * matrix.  Per super-block the rows' records come by LDS-DMA (two buffers;
+ * w columns 32 w .. 32 w + 31 of gate and of up.  Per super-block the rows' records come by LDS-DMA (two buffers;
  * one load moves a pair of chunks of all 32 rows, which an operand read then
  * takes as 1 KB in a run) and are shared by the waves; a lane's columns' raw
  * blocks load straight into registers, each matrix's next super-block once
@@ -325,14 +331,14 @@ __device__ static inline int km_item(int id, int items)
  * the weights' bytes come next.  32 rows a tile: 64 need 256 registers of
  * accumulators, and the experts of a prompt average 10 to 60 rows.
  */
-template <int WT, bool MOE, int NW>
+template <int WT, int NW>
 __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 	const uint8_t *__restrict__ W, const uint8_t *__restrict__ W2, size_t stride,
 	const int *__restrict__ rows, const int *__restrict__ tile_e, int Tmax,
-	const uint8_t *__restrict__ rec, const float *__restrict__ scale, int topk, int T, int K,
-	int N, const float *__restrict__ add, int add_rows, float *__restrict__ out)
+	const uint8_t *__restrict__ rec, const float *__restrict__ scale, int topk, int K, int N,
+	float *__restrict__ out)
 {
-	constexpr int BY = kqb<WT>::BYTES, NC = MOE ? 2 : 1;
+	constexpr int BY = kqb<WT>::BYTES, NC = 2, LR = KM_LROW;
 	extern __shared__ __attribute__((aligned(16))) uint8_t km_lds[];
 	uint8_t *s_a = km_lds;                                   /* [2][34][32] chunks */
 	float *s_yd = (float *)(km_lds + 2 * 34 * KM_LROW);      /* [nb][32] */
@@ -340,21 +346,19 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 	const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
 	const int m = lane & 31, h = lane >> 5;
 	const int cbs = (N + NW * 32 - 1) / (NW * 32);
-	const int ntiles = MOE ? tile_e[Tmax] : (T + KM_ROWS - 1) / KM_ROWS;
+	const int ntiles = tile_e[Tmax];
 	const int item = km_item(blockIdx.x, ntiles * cbs);
 	if (item < 0)
 		return; /* the whole workgroup */
 	const int tile = item % ntiles, cb = item / ntiles;
 	const int col = cb * (NW * 32) + wave * 32 + m;
-	const size_t eo = MOE ? (size_t)tile_e[tile] * stride : 0;
+	const size_t eo = (size_t)tile_e[tile] * stride;
 	/* columns past N repeat the last one (never stored) */
 	const size_t co = eo + (size_t)min(col, N - 1) * nb * BY;
 	const uint8_t *wp[2] = {W + co, W2 + co};
 
 	/* row r of the tile's token */
 	auto token = [&](int r) {
-		if (!MOE)
-			return min(tile * KM_ROWS + r, T - 1);
 		const int p = rows[tile * KM_ROWS + r];
 		return p < 0 ? 0 : p / topk; /* padding rows compute token 0's */
 	};
@@ -399,9 +403,9 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 		for (int c = 0; c < NC; c++) {
 			floatx16 S1, S2;
 			w[c].pin(); /* not ahead of the other matrix's loads */
-			km_mins(w[c], sa, m, h, yd, accm[c]);
+			km_mins<LR>(w[c], sa, m, h, yd, accm[c]);
 			__builtin_amdgcn_sched_barrier(0);
-			km_sums(w[c], sa, m, h, S1, S2);
+			km_sums<LR>(w[c], sa, m, h, S1, S2);
 			km_step(w[c], S1, S2, yd, acc[c]);
 			__builtin_amdgcn_sched_barrier(0);
 			/* the next super-block's, into the registers just read */
@@ -415,13 +419,154 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 	for (int j = 0; j < 16; j++) {
 		const int r = tile * KM_ROWS + 8 * (j / 4) + 4 * h + j % 4;
 		const float g = WT == 3 ? acc[0][j] + accm[0][j] : acc[0][j];
-		if constexpr (MOE) {
-			const float u = WT == 3 ? acc[1][j] + accm[1][j] : acc[1][j];
-			out[(size_t)r * N + col] = (g / (1.0f + moe_expf(-g))) * u;
-		} else if (r < T) {
-			const size_t o = (size_t)r * N + col;
-			out[o] = (add ? add[add_rows ? o : (size_t)col] : 0.0f) + g;
+		const float u = WT == 3 ? acc[1][j] + accm[1][j] : acc[1][j];
+		out[(size_t)r * N + col] = (g / (1.0f + moe_expf(-g))) * u;
+	}
+}
+
+/* ------------------------------------------------------------------ */
+/* the dense product                                                    */
+/* ------------------------------------------------------------------ */
+
+/*
+ * quantize_row_q8 (quant.c:627-654) of one super-block of a tile's 32 rows
+ * into operand chunks at sa and scales at yd, by 256 threads: eight a row,
+ * thread i of a row holding its float4s i, i + 8, ... (v[j]: values 4 (i + 8 j)
+ * on), so that a load reads 128-byte runs.  The value of largest magnitude
+ * comes from the signed extremes; only where both magnitudes are equal does
+ * the index decide (the first wins).
+ */
+__device__ static inline void kq_stage(const float4 (&v)[8], uint8_t *sa, float *yd, int row, int i)
+{
+	constexpr int LR = KM_LROW_Q;
+	float hi = 0.0f, lo = 0.0f;
+#pragma unroll
+	for (int j = 0; j < 8; j++) {
+		hi = fmaxf(fmaxf(fmaxf(hi, v[j].x), fmaxf(v[j].y, v[j].z)), v[j].w);
+		lo = fminf(fminf(fminf(lo, v[j].x), fminf(v[j].y, v[j].z)), v[j].w);
+	}
+#pragma unroll
+	for (int off = 1; off < 8; off <<= 1) {
+		hi = fmaxf(hi, __shfl_xor(hi, off, WAVE));
+		lo = fminf(lo, __shfl_xor(lo, off, WAVE));
+	}
+	float bv = hi > -lo ? hi : lo;
+	if (hi == -lo && hi > 0.0f) { /* the eight threads of a row agree */
+		int key = 0x7fffffff;
+#pragma unroll
+		for (int j = 7; j >= 0; j--) {
+			const float e[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+			for (int k = 3; k >= 0; k--)
+				if (fabsf(e[k]) == hi)
+					key = (4 * (i + 8 * j) + k) * 2 + (e[k] < 0.0f);
 		}
+#pragma unroll
+		for (int off = 1; off < 8; off <<= 1)
+			key = min(key, __shfl_xor(key, off, WAVE));
+		bv = key & 1 ? lo : hi;
+	}
+	const bool zero = bv == 0.0f;
+	const float iscale = zero ? 0.0f : -127.0f / bv;
+	const int h = i >> 2, u = (i >> 1) & 1;
+#pragma unroll
+	for (int j = 0; j < 8; j++) {
+		const float e[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+		half4_t o;
+		int s = 0;
+#pragma unroll
+		for (int k = 0; k < 4; k++) {
+			int q = zero ? 0 : (int)roundf(iscale * e[k]);
+			q = q < 127 ? q : 127;
+			s += q;
+			/* values 0, 2, 1, 3: the order of a weight operand (k_kq_rec) */
+			o[k == 1 ? 2 : k == 2 ? 1 : k] = (_Float16)(float)(int8_t)(q & 0xff);
+		}
+		*(half4_t *)(sa + ((2 * j + u) * 2 + h) * LR + row * 16 + (i & 1) * 8) = o;
+		s += __shfl_xor(s, 1, WAVE);
+		s += __shfl_xor(s, 2, WAVE);
+		/* sum i / 4 + 2 j of 16 values, finite in f16 as in k_kq_rec */
+		if ((i & 3) == 0)
+			*(_Float16 *)(sa + (32 + (j >> 2)) * LR + row * 16 + 2 * ((h + 2 * j) & 7)) =
+				(_Float16)(float)max(-2048, min(2048, s));
+	}
+	if (i == 0)
+		yd[row] = zero ? 0.0f : 1.0f / iscale;
+}
+
+#define KD_WAVES 4
+
+/*
+ * out = add + x . W^T for T tokens: a workgroup takes a tile of 32 tokens and
+ * 128 columns, as k_kq_mm takes one matrix, but quantizes its tokens itself
+ * into the LDS buffer the next super-block is read from: a call then holds no
+ * scratch memory, so calls on one matrix may overlap and be captured.  The
+ * quantization is done again for every 128 columns; it costs about as many
+ * VALU cycles as the operands of one wave's 32 columns.
+ *
+ * Bound: the VALU, in series with the MFMAs where a call has fewer than two
+ * workgroups per CU.  4096 x 4096 Q4_K: 77 tokens 384 -> 47 us, 333 tokens
+ * 1771 -> 71 us against the per-token product (whose groups of tokens re-read
+ * and re-unpack every weight); Q6_K 390 -> 78 and 1772 -> 115 us; 4096 x 14336
+ * Q4_K, 77 tokens: 2132 -> 154 us.
+ */
+template <int WT>
+__global__ __launch_bounds__(KD_WAVES * WAVE, 2) void k_kq_dense(
+	const uint8_t *__restrict__ W, const float *__restrict__ x, int T, int K, int N,
+	const float *__restrict__ add, int add_rows, float *__restrict__ out)
+{
+	constexpr int BY = kqb<WT>::BYTES, LR = KM_LROW_Q;
+	__shared__ __attribute__((aligned(16))) uint8_t s_a[2][34 * LR];
+	__shared__ __attribute__((aligned(16))) float s_yd[2][KM_ROWS];
+	const int nb = K / 256, tid = threadIdx.x, lane = tid % WAVE;
+	const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+	const int m = lane & 31, h = lane >> 5;
+	const int ntiles = (T + KM_ROWS - 1) / KM_ROWS, cbs = (N + KD_WAVES * 32 - 1) / (KD_WAVES * 32);
+	const int item = km_item(blockIdx.x, ntiles * cbs);
+	if (item < 0)
+		return; /* the whole workgroup */
+	const int tile = item % ntiles, col = item / ntiles * (KD_WAVES * 32) + wave * 32 + m;
+	/* columns past N repeat the last one, rows past T the last token (never stored) */
+	const uint8_t *wp = W + (size_t)min(col, N - 1) * nb * BY;
+	const int row = tid >> 3, i = tid & 7;
+	const float4 *xp = (const float4 *)(x + (size_t)min(tile * KM_ROWS + row, T - 1) * K) + i;
+	float4 v[8];
+	kmw<WT> w;
+	floatx16 acc = {}, accm = {};
+#pragma unroll
+	for (int j = 0; j < 8; j++)
+		v[j] = xp[8 * j];
+	w.load(wp, h);
+	kq_stage(v, s_a[0], s_yd[0], row, i);
+	for (int sb = 0; sb < nb; sb++) {
+		const int nx = min(sb + 1, nb - 1), b = sb & 1;
+		__syncthreads(); /* buffer b is whole, the other one is free */
+#pragma unroll
+		for (int j = 0; j < 8; j++)
+			v[j] = xp[(size_t)nx * 64 + 8 * j];
+		const floatx4 *yd = (const floatx4 *)(s_yd[b] + 4 * h);
+		floatx16 S1, S2;
+		km_mins<LR>(w, s_a[b], m, h, yd, accm);
+		__builtin_amdgcn_sched_barrier(0);
+		km_sums<LR>(w, s_a[b], m, h, S1, S2);
+		km_step(w, S1, S2, yd, acc);
+		__builtin_amdgcn_sched_barrier(0);
+		/* the next super-block's, into the registers just read */
+		w.load(wp + (size_t)nx * BY, h);
+		__builtin_amdgcn_sched_barrier(0);
+		if (sb + 1 < nb)
+			kq_stage(v, s_a[b ^ 1], s_yd[b ^ 1], row, i);
+	}
+	if (col >= N)
+		return;
+#pragma unroll
+	for (int j = 0; j < 16; j++) {
+		const int r = tile * KM_ROWS + 8 * (j / 4) + 4 * h + j % 4;
+		if (r >= T)
+			continue;
+		const size_t o = (size_t)r * N + col;
+		out[o] = (add ? add[add_rows ? o : (size_t)col] : 0.0f) +
+			 (WT == 3 ? acc[j] + accm[j] : acc[j]);
 	}
 }
 
@@ -661,18 +806,49 @@ extern "C" int moe_launch_kq_grouped(int gt, int dt, const uint8_t *gate, const 
 	const unsigned gd = (unsigned)(((long long)Tmax * (E / KW_COLS) + 7) / 8 * 8);
 	const float *scale = rec_scales(rec, (size_t)T, (size_t)E);
 	if (gt == 3)
-		hipLaunchKernelGGL((k_kq_mm<3, true, 4>), dim3(gg), dim3(256), km_lds_bytes(E), s, gate,
-				   up, gu_stride, rows, tile_e, Tmax, (const uint8_t *)rec, scale, topk,
-				   T, E, EI, (const float *)nullptr, 0, h);
+		hipLaunchKernelGGL((k_kq_mm<3, 4>), dim3(gg), dim3(256), km_lds_bytes(E), s, gate, up,
+				   gu_stride, rows, tile_e, Tmax, (const uint8_t *)rec, scale, topk, E,
+				   EI, h);
 	else
-		hipLaunchKernelGGL((k_kq_mm<5, true, 4>), dim3(gg), dim3(256), km_lds_bytes(E), s, gate,
-				   up, gu_stride, rows, tile_e, Tmax, (const uint8_t *)rec, scale, topk,
-				   T, E, EI, (const float *)nullptr, 0, h);
+		hipLaunchKernelGGL((k_kq_mm<5, 4>), dim3(gg), dim3(256), km_lds_bytes(E), s, gate, up,
+				   gu_stride, rows, tile_e, Tmax, (const uint8_t *)rec, scale, topk, E,
+				   EI, h);
 	if (dt == 3)
 		hipLaunchKernelGGL(k_kq_down_mm<3>, dim3(gd), dim3(256), 0, s, down, dn_stride, rows,
 				   tile_e, Tmax, h, E, EI, y);
 	else
 		hipLaunchKernelGGL(k_kq_down_mm<5>, dim3(gd), dim3(256), 0, s, down, dn_stride, rows,
 				   tile_e, Tmax, h, E, EI, y);
+	return (int)hipGetLastError();
+}
+
+/* A tile costs the same for 1 and for 32 tokens, the per-token product grows
+ * with T.  Where they cross, per-token / tile in us: Q4_K 4096 x 4096 T = 8
+ * 45.0 / 45.5, T = 12 63.6 / 45.8; 2048 x 2048 T = 8 23.7 / 24.5, T = 12
+ * 35.0 / 24.9; Q6_K 4096 x 4096 T = 12 65.3 / 76.5, T = 16 84.0 / 76.4; 2048 x
+ * 2048 T = 12 38.6 / 39.3, T = 16 49.0 / 39.3.  Matrices whose 128-row blocks
+ * fill half the chip or more cross earlier: Q4_K 50304 x 2048 T = 7 46.5 /
+ * 38, 32000 x 4096 T = 7 90 / 50; Q6_K T = 8 60.1 / 59 and 93 / 87, T = 9 78 /
+ * 59 and 119 / 87 */
+extern "C" int moe_kq_dense_better(int wtype, size_t N, size_t T)
+{
+	if (N >= 16384)
+		return T >= (wtype == 3 ? 7 : 9);
+	return T >= (wtype == 3 ? 9 : 14);
+}
+
+extern "C" int moe_launch_kq_dense(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
+				   const float *add, int add_rows, float *out, void *stream)
+{
+	const long long items = (long long)((T + KM_ROWS - 1) / KM_ROWS) *
+				((N + KD_WAVES * 32 - 1) / (KD_WAVES * 32));
+	if ((wtype != 3 && wtype != 5) || N < 1 || T < 1 || K < 256 || K % 256 || items > 0x7fffff00ll)
+		return (int)hipErrorInvalidValue;
+	const dim3 grid((unsigned)((items + 7) / 8 * 8)), blk(KD_WAVES * WAVE);
+	hipStream_t s = (hipStream_t)stream;
+	if (wtype == 3)
+		hipLaunchKernelGGL(k_kq_dense<3>, grid, blk, 0, s, W, x, T, K, N, add, add_rows, out);
+	else
+		hipLaunchKernelGGL(k_kq_dense<5>, grid, blk, 0, s, W, x, T, K, N, add, add_rows, out);
 	return (int)hipGetLastError();
 }

@@ -141,6 +141,12 @@ int moe_launch_kq_grouped(int gt, int dt, const uint8_t *gate, const uint8_t *up
                           const uint8_t *down, size_t gu_stride, size_t dn_stride,
                           const int *rows, const int *tile_e, int Tmax, const void *rec,
                           float *h, float *y, int T, int topk, int E, int EI, void *stream);
+/* The dense product of several tokens on the matrix cores (kq_grouped.hip):
+ * moe_launch_kq_gemv's bits, without scratch memory.  moe_kq_dense_better:
+ * whether it is the faster one for N rows, T tokens. */
+int moe_kq_dense_better(int wtype, size_t N, size_t T);
+int moe_launch_kq_dense(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
+                        const float *add, int add_rows, float *out, void *stream);
 /* quantize_row_q8 of T rows of K values: d[T][K/256], qs[T][K], bsums[T][K/256][16] */
 int moe_launch_q8k_quantize(const float *x, int T, int K, float *d, int8_t *qs,
                             int16_t *bsums, void *stream);
