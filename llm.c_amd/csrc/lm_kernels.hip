@@ -1165,8 +1165,11 @@ __global__ __launch_bounds__(LM_NT) void k_lm_pf_qk(const float *__restrict__ qk
 	}
 }
 
-#define PF_QB 64 /* query rows of a prefill attention workgroup */
-#define PF_KB 64 /* cache rows per step of its key loop */
+#define PF_QB 16    /* query rows of a prefill attention workgroup */
+#define PF_KB 32    /* cache rows per step of a wave's key loop */
+#define PF_WAVES 4
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 /*
  * k_lm_pf_attn: query head h of rows q0 .. q0 + PF_QB - 1 of sequence z
@@ -1178,119 +1181,146 @@ __global__ __launch_bounds__(LM_NT) void k_lm_pf_qk(const float *__restrict__ qk
  * * scale (Mixtral); the softmax runs online over blocks of PF_KB rows
  * (each block's maximum, the running sum rescaled), as flash_attention
  * does (nn.c:570-641), with a fully masked prefix taken as weight 0 rather
- * than exp(-inf - -inf).  Thread (row qi = tid / 4, quarter u = tid % 4)
- * holds dims 32u .. 32u + 31 of the row's q and of its output; the four
- * quarters' partial dots meet in two lane shuffles.
+ * than exp(-inf - -inf).
+ *
+ * Both products run on v_mfma_f32_16x16x4_f32: fp32 operands and sums.  The
+ * waves take every PF_WAVES-th block of rows, each with its own maximum,
+ * sum and output, and meet in LDS at the end, so the key loop has no
+ * barrier and no shared memory.  Lane (n = lane % 16, g = lane / 16) holds
+ * query n throughout: the scores are computed transposed (A = k rows, B =
+ * q), so element j of a result is row 4g + j of the block against query n,
+ * which is where the second product (A = v transposed, B = the weights)
+ * wants its operand when MFMA j takes the rows 4g + j, g < 4, and the
+ * maximum, sum and rescaling are one value per lane.  The k dims of MFMA
+ * 4c + e are 16c + 4g + e and the output dims of its tile 4b + e are 64b +
+ * 4m + e, so that every load is of 16 bytes in 64- or 256-byte runs.
+ *
+ * Bound: the fp32 matrix rate and, for short prompts, the last queries'
+ * serial key loop: 16 queries a workgroup and the loop split four ways
+ * (longest first) keep that to T / 128 steps.  512 rows, 16 heads: 327 ->
+ * 33 us against 64 queries a workgroup on the VALU; 16 sequences of 64
+ * rows, 32 heads: 95 -> 41 us.
  */
-__global__ __launch_bounds__(LM_NT) void k_lm_pf_attn(const float *__restrict__ qo,
-						      const float *__restrict__ kc,
-						      const float *__restrict__ vc,
-						      float *__restrict__ out, int H, int KH, int C,
-						      int size, int T, int window, float scale,
-						      int scale_mul, size_t cstride)
+__global__ __launch_bounds__(PF_WAVES * WAVE) void k_lm_pf_attn(
+	const float *__restrict__ qo, const float *__restrict__ kc, const float *__restrict__ vc,
+	float *__restrict__ out, int H, int KH, int C, int size, int T, int window, float scale,
+	int scale_mul, size_t cstride)
 {
-	constexpr int HL = LM_HLEN, RS = HL + 4, SS = PF_KB + 1;
-	static_assert(LM_NT == 4 * PF_QB, "four threads per query row");
-	__shared__ __attribute__((aligned(16))) float sk[PF_KB * RS], sv[PF_KB * RS];
-	/* a block's scores of each query row (kept in registers, unrolled, the
-	 * 64 scores and their operands spilled ~6.5 KB a lane to scratch) */
-	__shared__ float ssc[PF_QB * SS];
-	const int h = blockIdx.x, q0 = blockIdx.y * PF_QB, z = blockIdx.z;
+	constexpr int HL = LM_HLEN;
+	static_assert(HL == 128, "two 64-dim groups of a lane's 16-byte loads");
+	__shared__ __attribute__((aligned(16))) float s_o[PF_WAVES][PF_QB][HL + 4];
+	__shared__ float s_m[PF_WAVES][PF_QB], s_l[PF_WAVES][PF_QB];
+	const int h = blockIdx.x, z = blockIdx.z;
+	const int q0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * PF_QB; /* the longest first */
 	const int EQ = H * HL, kh = h / (H / KH);
-	const int tid = threadIdx.x, qi = tid / 4, u = tid % 4;
-	const int t = q0 + qi;
-	const bool live = t < T;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+	const int lane = threadIdx.x % WAVE, n = lane & 15, g = lane >> 4;
+	const int t = min(q0 + n, T - 1); /* rows past T repeat the last one (never stored) */
 	kc += (size_t)z * cstride + (size_t)kh * C * HL;
 	vc += (size_t)z * cstride + (size_t)kh * C * HL;
-	float qv[32], o[32];
+	floatx4 q[8], o[8];
 	{
-		const float4 *q4 = (const float4 *)(qo + ((size_t)z * T + (live ? t : 0)) * EQ +
-						    (size_t)h * HL + 32 * u);
+		const floatx4 *p = (const floatx4 *)(qo + ((size_t)z * T + t) * EQ + (size_t)h * HL) + g;
 #pragma unroll
-		for (int i = 0; i < 8; i++) {
-			const float4 v = q4[i];
-			qv[4 * i] = v.x;
-			qv[4 * i + 1] = v.y;
-			qv[4 * i + 2] = v.z;
-			qv[4 * i + 3] = v.w;
+		for (int c = 0; c < 8; c++) {
+			q[c] = p[4 * c];
+			o[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 		}
 	}
-#pragma unroll
-	for (int i = 0; i < 32; i++)
-		o[i] = 0.0f;
-	const int qa = size + t; /* this row's absolute position in the cache */
-	const int tlast = min(q0 + PF_QB, T) - 1;
-	const int jhi = size + tlast + 1; /* rows the block's last query sees */
+	const int qa = size + t; /* this query's absolute position in the cache */
+	const int jhi = size + min(q0 + PF_QB, T); /* rows the tile's last query sees */
 	const int jlo = window > 0 ? max(0, size + q0 - window + 1) : 0;
 	float m = -INFINITY, l = 0.0f;
-	for (int j0 = jlo; j0 < jhi; j0 += PF_KB) {
-		__syncthreads(); /* the previous block's readers are done */
-		for (int e = tid; e < PF_KB * HL / 4; e += LM_NT) {
-			const int jj = e / (HL / 4), c4 = e % (HL / 4);
-			float4 kv = {0.0f, 0.0f, 0.0f, 0.0f}, vv = kv;
-			if (j0 + jj < jhi) {
-				kv = ((const float4 *)(kc + (size_t)(j0 + jj) * HL))[c4];
-				vv = ((const float4 *)(vc + (size_t)(j0 + jj) * HL))[c4];
-			}
-			*(float4 *)(sk + jj * RS + 4 * c4) = kv;
-			*(float4 *)(sv + jj * RS + 4 * c4) = vv;
-		}
-		__syncthreads();
-		float *sc = ssc + qi * SS;
-#pragma unroll 2
-		for (int jj = 0; jj < PF_KB; jj++) {
-			const float4 *k4 = (const float4 *)(sk + jj * RS + 32 * u);
-			float a = 0.0f;
+	for (int j0 = jlo + wave * PF_KB; j0 < jhi; j0 += PF_WAVES * PF_KB) {
+		floatx4 s[2];
 #pragma unroll
-			for (int i = 0; i < 8; i++) {
-				const float4 kv = k4[i];
-				a = __builtin_fmaf(qv[4 * i], kv.x, a);
-				a = __builtin_fmaf(qv[4 * i + 1], kv.y, a);
-				a = __builtin_fmaf(qv[4 * i + 2], kv.z, a);
-				a = __builtin_fmaf(qv[4 * i + 3], kv.w, a);
-			}
-			a += __shfl_xor(a, 1, WAVE);
-			a += __shfl_xor(a, 2, WAVE);
-			const int j = j0 + jj;
-			const bool keep = j <= qa && (window <= 0 || qa - j < window);
-			if (u == 0)
-				sc[jj] = keep ? (scale_mul ? a * scale : a / scale) : -INFINITY;
+		for (int b = 0; b < 2; b++) { /* rows past jhi repeat the last one (masked) */
+			const floatx4 *kp =
+				(const floatx4 *)(kc + (size_t)min(j0 + 16 * b + n, jhi - 1) * HL) + g;
+			floatx4 k[8];
+#pragma unroll
+			for (int c = 0; c < 8; c++)
+				k[c] = kp[4 * c];
+			s[b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+			for (int c = 0; c < 8; c++)
+#pragma unroll
+				for (int e = 0; e < 4; e++)
+					s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c][e], q[c][e], s[b], 0, 0, 0);
 		}
-		__syncthreads(); /* the row's scores, from its quarter 0 */
+		floatx4 v[2][4][2];
+#pragma unroll
+		for (int b = 0; b < 2; b++)
+#pragma unroll
+			for (int j = 0; j < 4; j++) {
+				const floatx4 *vp = (const floatx4 *)(
+					vc + (size_t)min(j0 + 16 * b + 4 * g + j, jhi - 1) * HL) + n;
+				v[b][j][0] = vp[0];
+				v[b][j][1] = vp[16];
+			}
 		float mb = -INFINITY;
-#pragma unroll 8
-		for (int jj = 0; jj < PF_KB; jj++)
-			mb = fmaxf(mb, sc[jj]);
+#pragma unroll
+		for (int b = 0; b < 2; b++)
+#pragma unroll
+			for (int j = 0; j < 4; j++) {
+				const int r = j0 + 16 * b + 4 * g + j;
+				const bool keep = r <= qa && (window <= 0 || qa - r < window);
+				const float a = s[b][j];
+				s[b][j] = keep ? (scale_mul ? a * scale : a / scale) : -INFINITY;
+				mb = fmaxf(mb, s[b][j]);
+			}
+		mb = fmaxf(mb, __shfl_xor(mb, 16, WAVE));
+		mb = fmaxf(mb, __shfl_xor(mb, 32, WAVE));
 		const float mn = fmaxf(m, mb);
-		if (mn == -INFINITY)
-			continue; /* nothing of this row so far */
 		const float corr = m == -INFINITY ? 0.0f : moe_expf(m - mn);
 		l = l * corr;
 #pragma unroll
-		for (int i = 0; i < 32; i++)
-			o[i] = o[i] * corr;
-#pragma unroll 2
-		for (int jj = 0; jj < PF_KB; jj++) {
-			const float sj = sc[jj];
-			const float pj = sj == -INFINITY ? 0.0f : moe_expf(sj - mn);
-			l = l + pj;
-			const float4 *v4 = (const float4 *)(sv + jj * RS + 32 * u);
+		for (int c = 0; c < 8; c++)
+			o[c] = o[c] * corr;
 #pragma unroll
-			for (int i = 0; i < 8; i++) {
-				const float4 vv = v4[i];
-				o[4 * i] = __builtin_fmaf(pj, vv.x, o[4 * i]);
-				o[4 * i + 1] = __builtin_fmaf(pj, vv.y, o[4 * i + 1]);
-				o[4 * i + 2] = __builtin_fmaf(pj, vv.z, o[4 * i + 2]);
-				o[4 * i + 3] = __builtin_fmaf(pj, vv.w, o[4 * i + 3]);
+		for (int b = 0; b < 2; b++)
+#pragma unroll
+			for (int j = 0; j < 4; j++) {
+				const float p = s[b][j] == -INFINITY ? 0.0f : moe_expf(s[b][j] - mn);
+				l = l + p;
+#pragma unroll
+				for (int c = 0; c < 8; c++)
+					o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][j][c / 4][c % 4], p, o[c],
+										      0, 0, 0);
 			}
-		}
 		m = mn;
 	}
-	if (live) {
-		float4 *o4 = (float4 *)(out + ((size_t)z * T + t) * EQ + (size_t)h * HL + 32 * u);
+	l += __shfl_xor(l, 16, WAVE);
+	l += __shfl_xor(l, 32, WAVE);
+	if (g == 0) {
+		s_m[wave][n] = m;
+		s_l[wave][n] = l;
+	}
+	/* element j of tile c is dim 64 (c / 4) + 16 g + 4 j + c % 4 of query n */
 #pragma unroll
-		for (int i = 0; i < 8; i++)
-			o4[i] = float4{o[4 * i] / l, o[4 * i + 1] / l, o[4 * i + 2] / l, o[4 * i + 3] / l};
+	for (int b = 0; b < 2; b++)
+#pragma unroll
+		for (int j = 0; j < 4; j++)
+			*(floatx4 *)&s_o[wave][n][64 * b + 16 * g + 4 * j] =
+				floatx4{o[4 * b][j], o[4 * b + 1][j], o[4 * b + 2][j], o[4 * b + 3][j]};
+	__syncthreads();
+	/* the waves' parts: thread (query i / 32, dims 4 (i % 32) ..) */
+	for (int i = threadIdx.x; i < PF_QB * HL / 4; i += PF_WAVES * WAVE) {
+		const int qi = i / (HL / 4), d = 4 * (i % (HL / 4));
+		float mm = s_m[0][qi];
+#pragma unroll
+		for (int w = 1; w < PF_WAVES; w++)
+			mm = fmaxf(mm, s_m[w][qi]);
+		float sum = 0.0f;
+		floatx4 r = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+		for (int w = 0; w < PF_WAVES; w++) {
+			const float mw = s_m[w][qi], f = mw == -INFINITY ? 0.0f : moe_expf(mw - mm);
+			sum = sum + f * s_l[w][qi];
+			r = r + f * *(const floatx4 *)&s_o[w][qi][d];
+		}
+		if (q0 + qi < T)
+			*(floatx4 *)(out + ((size_t)z * T + q0 + qi) * EQ + (size_t)h * HL + d) = r / sum;
 	}
 }
 
@@ -1520,7 +1550,7 @@ extern "C" int lm_launch_pf_attn(const float *qo, const float *kc, const float *
 	if (T < 1 || nseq < 1 || nseq > 65535 || KH < 1 || H % KH || size < 0 || size + T > C ||
 	    (T + PF_QB - 1) / PF_QB > 65535)
 		return (int)hipErrorInvalidValue;
-	hipLaunchKernelGGL(k_lm_pf_attn, dim3(H, (T + PF_QB - 1) / PF_QB, nseq), dim3(LM_NT), 0,
+	hipLaunchKernelGGL(k_lm_pf_attn, dim3(H, (T + PF_QB - 1) / PF_QB, nseq), dim3(PF_WAVES * WAVE), 0,
 			   (hipStream_t)stream, qo, kc, vc, out, H, KH, C, size, T, window, scale,
 			   scale_mul, cstride);
 	return (int)hipGetLastError();
