@@ -283,8 +283,8 @@ hip_moe_qmat *hip_moe_qmat_upload(const void *qdata, int wtype, size_t N, size_t
  * absolute error per output within 2^-24 * (32 (127 + c) + 31 c + 64 * 255)
  * * (sum over blocks of |d| * sum |x|) to first order; ~1e-6 relative L2 on
  * zero-mean activations.  Several tokens (T >= 2) of a Q8_0/Q4_0 matrix run
- * on the matrix cores instead: each 32-value token block scaled by a power
- * of two and split into two f16 parts (~22 bits together), the quants
+ * on the matrix cores instead: each token's 32 (few tokens) or 128 values
+ * scaled by a power of two and split into two f16 parts (~22 bits together), the quants
  * unscaled (exact in f16), the block scale applied per block in fp32, so the
  * outputs keep fp32 accuracy (~1e-7 relative, summation order only).
  * Q4_K/Q6_K matrices take the reference's Q8_K
@@ -301,7 +301,7 @@ int hip_moe_qmat_mul(hip_moe_qmat *W, const float *x, size_t T, const float *add
  * without waiting (NULL = the library's stream for W's device).  It
  * allocates nothing: the matrix-core form's token buffer, made at upload,
  * holds 64 tokens (more after a host call of more tokens); calls with more
- * take the per-token product.  Calls that overlap on one matrix race on
+ * take a form without one.  Calls that overlap on one matrix race on
  * that buffer.  A host call (hip_moe_qmat_mul) with more tokens than the
  * buffer holds replaces it (after waiting for the device): HIP graphs
  * captured earlier with this function on W name the freed buffer and must

@@ -917,7 +917,10 @@ static int rows_product(hip_lm *M, const uint8_t *W, int N, int K, const float *
 			const float *add, float *out, hipStream_t s)
 {
 	const int wt = M->wtype;
-	if (moe_qmm_supported(wt, K))
+	if (moe_qmm_supported(wt, K) && moe_qmm_tile_better(N, T))
+		LCHK(moe_launch_qmm_tile(wt, W, N, K, x, T, add, add != NULL, out, s),
+		     "prefill product");
+	else if (moe_qmm_supported(wt, K))
 		LCHK(moe_launch_qmm(wt, W, N, K, x, T, add, add != NULL, out, M->d_pf_split, s),
 		     "prefill product");
 	else
@@ -1417,7 +1420,9 @@ static int batch_product(hip_lm_batch *B, const uint8_t *W, int N, int K, const 
 			 const float *add, float *out)
 {
 	const int wt = B->M->wtype, S = (int)B->S;
-	if (moe_qmm_supported(wt, K)) {
+	if (moe_qmm_supported(wt, K) && moe_qmm_tile_better(N, S)) {
+		LCHK(moe_launch_qmm_tile(wt, W, N, K, x, S, add, add != NULL, out, B->stream), "product");
+	} else if (moe_qmm_supported(wt, K)) {
 		LCHK(moe_launch_qmm(wt, W, N, K, x, S, add, add != NULL, out, B->d_split, B->stream),
 		     "product");
 	} else {
@@ -1452,7 +1457,8 @@ static int batch_step(hip_lm_batch *B, int head, int nact)
 		 * product leaves partial sums, one launch adds them (the reduce's
 		 * order), adds h0 and normalises */
 		const int EQ = (int)M->EQ;
-		if (moe_qmm_supported(wt, EQ) && moe_qmm_stretches(EQ) > 1) {
+		if (moe_qmm_supported(wt, EQ) && moe_qmm_stretches(EQ) > 1 &&
+		    !moe_qmm_tile_better(E, S)) {
 			LCHK(moe_launch_qmm_parts(wt, y->wo, E, EQ, B->d_attn, S, B->d_split, s),
 			     "output product");
 			LCHK(lm_launch_norm_parts(S, E, B->d_split, moe_qmm_stretches(EQ), (size_t)S * E,

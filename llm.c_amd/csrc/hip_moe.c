@@ -1048,8 +1048,8 @@ struct hip_moe_qmat {
 };
 
 /* tokens the matrix-core product's split buffer holds from upload on (the
- * device entry point allocates nothing: more tokens take the per-token
- * product) */
+ * device entry point allocates nothing: more tokens take the tiles, which
+ * need none) */
 #define QMAT_SPLIT_T 64
 
 /* the matrix-core product's partial sums for up to T tokens (the old ones
@@ -1172,8 +1172,13 @@ int hip_moe_qmat_mul_dev(const hip_moe_qmat *W, const float *d_x, size_t T,
 		LCHK(moe_launch_kq_gemv(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 					add_len == T * W->N, d_out, T == 1 ? W->grid1 : W->grid, s),
 		     "kq_gemv");
-	} else if (T > 1 && W->qmm && T <= W->split_T) {
-		/* several tokens: on the matrix cores, at fp32 accuracy */
+	} else if (T > 1 && W->qmm &&
+		   (T > W->split_T || moe_qmm_tile_better((int)W->N, (int)T))) {
+		/* several tokens: on the matrix cores, at fp32 accuracy; in tiles of
+		 * 64 tokens where those are faster or the split buffer holds fewer */
+		LCHK(moe_launch_qmm_tile(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
+					 add_len == T * W->N, d_out, s), "qmm_tile");
+	} else if (T > 1 && W->qmm) {
 		LCHK(moe_launch_qmm(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 				    add_len == T * W->N, d_out, W->d_split, s), "qmm");
 	} else
@@ -1208,7 +1213,8 @@ int hip_moe_qmat_mul(hip_moe_qmat *W, const float *x, size_t T, const float *add
 		HIPCHK(hipMalloc((void **)&W->d_out, T * W->N * sizeof(float)), "hipMalloc(out)");
 		W->cap_T = T;
 	}
-	if (W->qmm && T > W->split_T) { /* the host entry point may allocate */
+	/* the host entry point may allocate */
+	if (W->qmm && T > W->split_T && !moe_qmm_tile_better((int)W->N, (int)T)) {
 		/* device-pointer calls on any stream may still read the old buffer */
 		HIPCHK(hipDeviceSynchronize(), "synchronize");
 		if (!qmat_split_alloc(W, T))

@@ -59,6 +59,19 @@ __device__ static inline void dma_dwordx4(const void *sbase, u32 voff, u32 lds)
 		     : "memory");
 }
 
+/* the same, 4 bytes a lane */
+__device__ static inline void dma_dword(const void *sbase, u32 voff, u32 lds)
+{
+	const uint64_t b = (uint64_t)(uintptr_t)sbase;
+	const uint64_t bs = (uint64_t)(u32)__builtin_amdgcn_readfirstlane((int)(u32)b) |
+			    ((uint64_t)(u32)__builtin_amdgcn_readfirstlane((int)(u32)(b >> 32)) << 32);
+	asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1"
+		     :
+		     : "v"(voff), "s"((const void *)(uintptr_t)bs),
+		       "{m0}"(__builtin_amdgcn_readfirstlane(lds))
+		     : "memory");
+}
+
 /* wait until at most N of this wave's vector memory operations are pending
  * (loads return in order, so the older ones are then complete) */
 template <int N>
