@@ -85,6 +85,8 @@ struct hip_lm {
 	unsigned graph_gen; /* the MoE layers' scratch generation the graphs name */
 	unsigned path_gen;  /* forced MoE path changes (hip_lm_set_moe_path) */
 	hipEvent_t ev0, ev1;
+	/* pinned: lm_launch_report's words (16), then a row of logits */
+	int *h_io;
 
 	/* prefill: a prompt of up to pf_cap rows in one forward, rows [T][.] */
 	size_t pf_cap, pf_heads; /* rows, and sequences whose last rows take the lm_head */
@@ -260,6 +262,8 @@ void hip_lm_free(hip_lm *M)
 			M->d_st, M->d_prompt, M->d_tokens};
 	for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
 		hipFree(bufs[i]);
+	if (M->h_io)
+		hipHostFree(M->h_io);
 	if (M->ev0)
 		hipEventDestroy(M->ev0);
 	if (M->ev1)
@@ -410,6 +414,7 @@ hip_lm *hip_lm_upload(const hip_lm_desc *d)
 
 	HIPCHK(hipGetDevice(&M->device), "hipGetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&M->stream, hipStreamNonBlocking), "hipStreamCreate");
+	HIPCHK(hipHostMalloc((void **)&M->h_io, (16 + M->V) * sizeof(float), 0), "hipHostMalloc");
 	HIPCHK(hipEventCreate(&M->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&M->ev1), "hipEventCreate");
 
@@ -807,10 +812,15 @@ fail:
 /* set the device counters for a run of n_prompt prompt steps */
 static int start_run(hip_lm *M, const int *prompt, size_t n_prompt)
 {
-	/* earlier steps on the (non-blocking) stream read these buffers */
-	HIPCHK(hipStreamSynchronize(M->stream), "synchronize");
 	M->st.step = 0;
 	M->st.n_prompt = (int)n_prompt;
+	if (n_prompt <= LM_SET_IDS) {
+		LCHK(lm_launch_set_state(M->d_st, &M->st, M->d_prompt, prompt, (int)n_prompt, M->stream),
+		     "set state");
+		return 1;
+	}
+	/* earlier steps on the (non-blocking) stream read these buffers */
+	HIPCHK(hipStreamSynchronize(M->stream), "synchronize");
 	if (n_prompt)
 		HIPCHK(hipMemcpy(M->d_prompt, prompt, n_prompt * sizeof(int), hipMemcpyHostToDevice),
 		       "copy prompt");
@@ -828,11 +838,31 @@ static void advance_host(hip_lm *M)
 	M->st.size++;
 }
 
+/* lm_launch_report of st and every MoE layer's error word on `s`; 0 (nothing
+ * enqueued, or a launch error) where the words have to be read one by one */
+static int enqueue_report(const hip_lm *M, const LmState *st, const int *btok, size_t nseq, int *out,
+			  hipStream_t s)
+{
+	const uint32_t *err[LM_REPORT_LAYERS];
+	if (M->L > LM_REPORT_LAYERS)
+		return 0;
+	for (size_t l = 0; l < M->L; l++)
+		if (!moe_err_word(M->ly[l].moe, &err[l]))
+			return 0;
+	return lm_launch_report(st, btok, (int)nseq, err, (int)M->L, out, s) == 0;
+}
+
 /* after the stream drains: a bounded wait of a gather or of a MoE layer's
- * decode kernel that ran out makes the run's results invalid */
+ * decode kernel that ran out makes the run's results invalid.  All error
+ * words come back in one launch and one wait (a copy each took 20 us). */
 static int check_errors(hip_lm *M, const char *what)
 {
 	int err = 0;
+	if (enqueue_report(M, M->d_st, NULL, 0, M->h_io, M->stream)) {
+		HIPCHK(hipStreamSynchronize(M->stream), "synchronize");
+		if (!M->h_io[0] && !M->h_io[1])
+			return 1;
+	}
 	HIPCHK(hipStreamSynchronize(M->stream), "synchronize");
 	HIPCHK(hipMemcpy(&err, &M->d_st->err, sizeof(int), hipMemcpyDeviceToHost), "read error");
 	if (err) {
@@ -849,9 +879,16 @@ static int check_errors(hip_lm *M, const char *what)
 			return 0;
 		}
 	}
+	HIPCHK(hipMemcpy(&M->h_io[2], &M->d_st->tok, sizeof(int), hipMemcpyDeviceToHost), "read pick");
 	return 1;
 fail:
 	return 0;
+}
+
+/* the pinned row of logits */
+static float *h_logits(const hip_lm *M)
+{
+	return (float *)(M->h_io + 16);
 }
 
 static int check_token(const hip_lm *M, int tok)
@@ -1051,15 +1088,17 @@ int hip_lm_prefill(hip_lm *M, const int *prompt, size_t n, float *logits, int *n
 		return 0;
 	M->st.pos += (int)n;
 	M->st.size += (int)n;
+	/* step and prompt counters belong to a run; the device's token stays */
+	LCHK(lm_launch_set_state(M->d_st, &M->st, NULL, NULL, 0, M->stream), "set state");
+	if (logits)
+		HIPCHK(hipMemcpyAsync(h_logits(M), M->d_logits, M->V * 4, hipMemcpyDeviceToHost,
+				      M->stream), "copy logits");
 	if (!check_errors(M, "lm_prefill"))
 		return 0;
-	/* step and prompt counters belong to a run; the device's token stays */
-	HIPCHK(hipMemcpy(M->d_st, &M->st, 4 * sizeof(int), hipMemcpyHostToDevice), "set state");
 	if (logits)
-		HIPCHK(hipMemcpy(logits, M->d_logits, M->V * 4, hipMemcpyDeviceToHost), "copy logits");
+		memcpy(logits, h_logits(M), M->V * 4);
 	if (next)
-		HIPCHK(hipMemcpy(next, &M->d_st->tok, sizeof(int), hipMemcpyDeviceToHost),
-		       "read pick");
+		*next = M->h_io[2];
 	return 1;
 fail:
 	return 0;
@@ -1076,15 +1115,15 @@ int hip_lm_decode(hip_lm *M, int tok, float *logits, int *next)
 	    !enqueue_step(M, 1, lm_attn_active(M->st.size, (int)M->window)))
 		return 0;
 	advance_host(M);
+	if (logits)
+		HIPCHK(hipMemcpyAsync(h_logits(M), M->d_logits, M->V * 4, hipMemcpyDeviceToHost,
+				      M->stream), "copy logits");
 	if (!check_errors(M, "lm_decode"))
 		return 0;
 	if (logits)
-		HIPCHK(hipMemcpy(logits, M->d_logits, M->V * 4, hipMemcpyDeviceToHost), "copy logits");
-	if (next) {
-		LmState st;
-		HIPCHK(hipMemcpy(&st, M->d_st, sizeof(st), hipMemcpyDeviceToHost), "read state");
-		*next = st.tok;
-	}
+		memcpy(logits, h_logits(M), M->V * 4);
+	if (next)
+		*next = M->h_io[2];
 	return 1;
 fail:
 	return 0;
@@ -1142,8 +1181,8 @@ int hip_lm_generate(hip_lm *M, const int *prompt, size_t n_prompt, size_t n_gen,
 		M->st.size += (int)n_prompt;
 		/* the prefill kernels do not read these four (the pick writes the
 		 * token after them); the step graphs below do */
-		HIPCHK(hipMemcpy(M->d_st, &M->st, 4 * sizeof(int), hipMemcpyHostToDevice),
-		       "set state after prefill");
+		LCHK(lm_launch_set_state(M->d_st, &M->st, NULL, NULL, 0, M->stream),
+		     "set state after prefill");
 		first = n_prompt;
 	}
 	if (M->graph_gen != moe_gen(M)) {
@@ -1266,7 +1305,11 @@ struct hip_lm_batch {
 	hipGraphExec_t *g_body, *g_head;
 	unsigned graph_gen; /* the MoE layers' scratch generation the graphs name */
 	hipEvent_t ev0, ev1;
+	int *h_io;          /* pinned: lm_launch_report's words for S sequences */
+	float *h_logits;    /* pinned [S][V], NULL past BATCH_PINNED bytes */
 };
+
+#define BATCH_PINNED ((size_t)16 << 20)
 
 static size_t batch_cache_floats(const hip_lm *M)
 {
@@ -1296,6 +1339,10 @@ void hip_lm_batch_free(hip_lm_batch *B)
 			B->d_prompt, B->d_tokens, B->d_split};
 	for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
 		hipFree(bufs[i]);
+	if (B->h_io)
+		hipHostFree(B->h_io);
+	if (B->h_logits)
+		hipHostFree(B->h_logits);
 	if (B->ev0)
 		hipEventDestroy(B->ev0);
 	if (B->ev1)
@@ -1335,6 +1382,10 @@ hip_lm_batch *hip_lm_batch_new(hip_lm *M, size_t nseq)
 	const size_t part = S * M->H * (size_t)M->nch * (LM_HLEN + 2) * sizeof(uint64_t);
 	HIPCHK(hipSetDevice(M->device), "hipSetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking), "hipStreamCreate");
+	HIPCHK(hipHostMalloc((void **)&B->h_io, (LM_REPORT_WORDS + S) * sizeof(int), 0), "hipHostMalloc");
+	if (S * M->V * sizeof(float) <= BATCH_PINNED)
+		HIPCHK(hipHostMalloc((void **)&B->h_logits, S * M->V * sizeof(float), 0),
+		       "hipHostMalloc");
 	HIPCHK(hipEventCreate(&B->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&B->ev1), "hipEventCreate");
 	HIPCHK(hipMalloc((void **)&B->d_kc, cache), "hipMalloc(batch k caches)");
@@ -1514,9 +1565,14 @@ fail:
 
 static int batch_start(hip_lm_batch *B, const int *prompts, size_t n_prompt)
 {
-	HIPCHK(hipStreamSynchronize(B->stream), "synchronize");
 	B->st.step = 0;
 	B->st.n_prompt = (int)n_prompt;
+	if (n_prompt * B->S <= LM_SET_IDS) {
+		LCHK(lm_launch_set_state(B->d_st, &B->st, B->d_prompt, prompts, (int)(n_prompt * B->S),
+					 B->stream), "set state");
+		return 1;
+	}
+	HIPCHK(hipStreamSynchronize(B->stream), "synchronize");
 	HIPCHK(hipMemcpy(B->d_prompt, prompts, n_prompt * B->S * sizeof(int),
 			 hipMemcpyHostToDevice), "copy prompts");
 	HIPCHK(hipMemcpy(B->d_st, &B->st, 4 * sizeof(int), hipMemcpyHostToDevice), "set state");
@@ -1528,7 +1584,14 @@ fail:
 static int batch_errors(hip_lm_batch *B, const char *what)
 {
 	int err = 0;
+	if (enqueue_report(B->M, B->d_st, B->d_btok, B->S, B->h_io, B->stream)) {
+		HIPCHK(hipStreamSynchronize(B->stream), "synchronize");
+		if (!B->h_io[0] && !B->h_io[1])
+			return 1;
+	}
 	HIPCHK(hipStreamSynchronize(B->stream), "synchronize");
+	HIPCHK(hipMemcpy(B->h_io + LM_REPORT_WORDS, B->d_btok, B->S * sizeof(int),
+			 hipMemcpyDeviceToHost), "read picks");
 	HIPCHK(hipMemcpy(&err, &B->d_st->err, sizeof(int), hipMemcpyDeviceToHost), "read error");
 	if (err) {
 		const int zero = 0;
@@ -1569,14 +1632,18 @@ int hip_lm_batch_decode(hip_lm_batch *B, const int *toks, float *logits, int *ne
 	    !batch_step(B, 1, lm_attn_active(B->st.size, (int)B->M->window)))
 		return 0;
 	batch_advance(B);
+	const size_t lb = B->S * B->M->V * 4;
+	if (logits && B->h_logits)
+		HIPCHK(hipMemcpyAsync(B->h_logits, B->d_logits, lb, hipMemcpyDeviceToHost, B->stream),
+		       "copy logits");
 	if (!batch_errors(B, "lm_batch_decode"))
 		return 0;
-	if (logits)
-		HIPCHK(hipMemcpy(logits, B->d_logits, B->S * B->M->V * 4, hipMemcpyDeviceToHost),
-		       "copy logits");
+	if (logits && B->h_logits)
+		memcpy(logits, B->h_logits, lb);
+	else if (logits)
+		HIPCHK(hipMemcpy(logits, B->d_logits, lb, hipMemcpyDeviceToHost), "copy logits");
 	if (next)
-		HIPCHK(hipMemcpy(next, B->d_btok, B->S * sizeof(int), hipMemcpyDeviceToHost),
-		       "copy picks");
+		memcpy(next, B->h_io + LM_REPORT_WORDS, B->S * sizeof(int));
 	return 1;
 fail:
 	return 0;
@@ -1644,8 +1711,8 @@ int hip_lm_batch_generate(hip_lm_batch *B, const int *prompts, size_t n_prompt, 
 		B->st.pos += (int)n_prompt;
 		B->st.size += (int)n_prompt;
 		/* the prefills do not read the batch's state; the step graphs do */
-		HIPCHK(hipMemcpy(B->d_st, &B->st, 4 * sizeof(int), hipMemcpyHostToDevice),
-		       "set state after prefill");
+		LCHK(lm_launch_set_state(B->d_st, &B->st, NULL, NULL, 0, B->stream),
+		     "set state after prefill");
 		first = n_prompt;
 	}
 	if (B->graph_gen != moe_gen(M)) { /* another batch grew the layers' scratch */
@@ -1684,6 +1751,20 @@ int hip_lm_batch_generate(hip_lm_batch *B, const int *prompts, size_t n_prompt, 
 		*decode_ms = 0.0f;
 		if (n_gen)
 			HIPCHK(hipEventElapsedTime(decode_ms, B->ev0, B->ev1), "event time");
+	}
+	/* every sequence's tokens: one copy of all rows where they are few (a
+	 * copy a sequence took 20 us each) */
+	const size_t all = B->S * B->tokens_cap;
+	int *rows = all * sizeof(int) <= ((size_t)1 << 20) ? malloc(all * sizeof(int)) : NULL;
+	if (rows) {
+		const hipError_t e = hipMemcpy(rows, B->d_tokens, all * sizeof(int),
+					       hipMemcpyDeviceToHost);
+		for (size_t q = 0; e == hipSuccess && q < B->S; q++)
+			memcpy(tokens + q * (n_gen + 1), rows + q * B->tokens_cap + (n_prompt - 1),
+			       (n_gen + 1) * sizeof(int));
+		free(rows);
+		HIPCHK(e, "copy tokens");
+		return 1;
 	}
 	for (size_t q = 0; q < B->S; q++)
 		HIPCHK(hipMemcpy(tokens + q * (n_gen + 1), B->d_tokens + q * B->tokens_cap + (n_prompt - 1),

@@ -70,6 +70,9 @@ struct hip_moe_layer {
 	float *d_x, *d_out, *d_bias;
 	uint32_t *d_ids_io;
 	float *d_w_io;
+	/* pinned staging of host calls of a few tokens: x and the bias,
+	 * then out, ids, weights and the error word */
+	uint8_t *h_io;
 };
 
 static __thread char g_err[512];
@@ -227,6 +230,8 @@ void hip_moe_free(hip_moe_layer *L)
 	hipFree(L->d_bias);
 	hipFree(L->d_ids_io);
 	hipFree(L->d_w_io);
+	if (L->h_io)
+		hipHostFree(L->h_io);
 	free(L); /* L->stream is the device's shared stream: it stays */
 }
 
@@ -586,6 +591,12 @@ static int check_and_reset_static(int dev)
 	return (int)err;
 fail:
 	return -1;
+}
+
+int moe_err_word(const hip_moe_layer *L, const uint32_t **word)
+{
+	*word = L->d_sync ? L->d_sync + MOE_SYNC_ERR_WORD : NULL;
+	return !L->used_static;
 }
 
 int hip_moe_status(hip_moe_layer *L, void *stream)
@@ -977,6 +988,62 @@ fail:
 	return 0;
 }
 
+/* bytes of x of a host call that goes through the pinned staging: a few
+ * tokens, whose copies are all latency (more bytes are worth the copy
+ * engines) */
+#define IO_PINNED ((size_t)128 << 10)
+
+/*
+ * A host call of a few tokens: x and the bias go through pinned memory that
+ * one launch reads, and the results and the error word come back by one
+ * launch and one wait (five copies that the host waited for took 60 us of
+ * the call).  1 = done, 0 = error, -1 = not applicable.
+ */
+static int ffn_pinned(hip_moe_layer *L, const float *x, float *out, size_t T,
+		      const float *router_bias, uint32_t *ids_out, float *w_out)
+{
+	const size_t most = IO_PINNED / (L->E * sizeof(float)), P = T * L->topk;
+	if (T > most)
+		return -1;
+	/* per token: x, out, ids, weights; the bias and the error word */
+	const size_t in = most * L->E + L->NE, res = most * (L->E + 2 * L->topk) + 1;
+	if (!L->h_io) {
+		if (hipHostMalloc((void **)&L->h_io, (in + res) * sizeof(float), 0) != hipSuccess) {
+			L->h_io = NULL;
+			return -1;
+		}
+	}
+	hipStream_t s = L->stream;
+	float *hx = (float *)L->h_io, *hb = hx + most * L->E, *ho = hx + in;
+	uint32_t *hi = (uint32_t *)(ho + T * L->E), *he = hi + 2 * P;
+	memcpy(hx, x, T * L->E * sizeof(float));
+	if (router_bias)
+		memcpy(hb, router_bias, L->NE * sizeof(float));
+	const moe_seg to[2] = {{hx, L->d_x, T * L->E}, {hb, L->d_bias, router_bias ? L->NE : 0}};
+	LCHK(moe_launch_copy_segs(to, 2, s), "copy x");
+	if (!hip_moe_ffn_dev(L, L->d_x, L->d_out, T, router_bias ? L->d_bias : NULL, L->d_ids_io,
+			     L->d_w_io, s))
+		return 0;
+	*he = 0;
+	const moe_seg from[4] = {{L->d_out, ho, T * L->E},
+				 {L->d_ids_io, hi, ids_out ? P : 0},
+				 {L->d_w_io, hi + P, w_out ? P : 0},
+				 {L->d_sync ? L->d_sync + MOE_SYNC_ERR_WORD : NULL, he, L->d_sync ? 1 : 0}};
+	LCHK(moe_launch_copy_segs(from, 4, s), "copy results");
+	HIPCHK(hipStreamSynchronize(s), "synchronize");
+	memcpy(out, ho, T * L->E * sizeof(float));
+	if (ids_out)
+		memcpy(ids_out, hi, P * sizeof(uint32_t));
+	if (w_out)
+		memcpy(w_out, hi + P, P * sizeof(float));
+	/* a bounded wait inside the decode kernel ran out: report and reset */
+	if (*he && check_and_reset(L, s) != 0)
+		return 0;
+	return 1;
+fail:
+	return 0;
+}
+
 int hip_moe_ffn(hip_moe_layer *L, const float *x, float *out, size_t T,
 		const float *router_bias, uint32_t *ids_out, float *w_out)
 {
@@ -986,6 +1053,9 @@ int hip_moe_ffn(hip_moe_layer *L, const float *x, float *out, size_t T,
 	}
 	if (!check_T(T) || !ensure_io(L, T))
 		return 0;
+	const int done = ffn_pinned(L, x, out, T, router_bias, ids_out, w_out);
+	if (done >= 0)
+		return done;
 	hipStream_t s = L->stream;
 	HIPCHK(hipMemcpyAsync(L->d_x, x, T * L->E * sizeof(float), hipMemcpyHostToDevice, s),
 	       "copy x");

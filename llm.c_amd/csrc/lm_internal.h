@@ -20,6 +20,10 @@ extern "C" {
 #define LM_HEAD_SLOT 63    /* the lm_head's slot; layers use 0 .. 62 */
 #define LM_MAX_HEAD_WG 4096
 
+#define LM_SET_IDS 128      /* prompt ids lm_launch_set_state takes */
+#define LM_REPORT_LAYERS 64 /* MoE layers lm_launch_report looks at */
+#define LM_REPORT_WORDS 4   /* words before the sequences' picks */
+
 #define LM_ERR_GATHER 1    /* a gather's poll ran out */
 
 /* The step's counters in device memory, read by every step kernel so that
@@ -103,6 +107,13 @@ int lm_launch_head(int wtype, const uint8_t *W, int N, int K, const float *a, co
                    const float *w, float *out, uint64_t *best, LmState *st, int *tokens,
                    int grid, void *stream);
 int lm_launch_step_end(LmState *st, void *stream);
+/* the first four counters of *st, and n ids of its prompt (n may be 0) */
+int lm_launch_set_state(LmState *st, const LmState *from, int *prompt, const int *ids, int n,
+                        void *stream);
+/* out (pinned host memory): st->err, whether an err word (entries may be
+ * NULL) is set, st->tok, unused, then btok[0 .. nseq) */
+int lm_launch_report(const LmState *st, const int *btok, int nseq, const uint32_t *const *err,
+                     int layers, int *out, void *stream);
 /* nseq sequences in lockstep: x_out[s] = rms_norm(a[s] + b[s]) * w (b may
  * be NULL; a NULL: the embedding row of sequence s's step token, from
  * prompt[s][step] while the prompt lasts, then btok[s]); h_out[s] (may be

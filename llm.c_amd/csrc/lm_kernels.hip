@@ -818,6 +818,50 @@ __global__ void k_lm_step_end(LmState *st)
 	}
 }
 
+/* the host's four counters (the others stay the device's) and the ids of a
+ * run's prompt, from the launch's arguments: ordered by the stream, without
+ * a copy that the host waits for */
+struct LmSet {
+	int st[4], n, ids[LM_SET_IDS];
+};
+
+__global__ __launch_bounds__(LM_SET_IDS) void k_lm_set_state(LmState *st, int *prompt, LmSet a)
+{
+	const int i = threadIdx.x;
+	if (i < a.n)
+		prompt[i] = a.ids[i];
+	if (i == 0) {
+		st->step = a.st[0];
+		st->n_prompt = a.st[1];
+		st->pos = a.st[2];
+		st->size = a.st[3];
+	}
+}
+
+/* what the host reads after a call, into its pinned words: the step kernels'
+ * error, any MoE layer's, the last pick, then each sequence's */
+struct LmReport {
+	const uint32_t *err[LM_REPORT_LAYERS];
+	int layers;
+};
+
+__global__ __launch_bounds__(256) void k_lm_report(const LmState *st, const int *btok, int nseq,
+						   LmReport a, int *out)
+{
+	int bad = 0;
+	for (int i = threadIdx.x; i < a.layers; i += 256)
+		if (a.err[i] && *a.err[i])
+			bad = 1;
+	bad = __syncthreads_or(bad);
+	for (int i = threadIdx.x; i < nseq; i += 256)
+		out[LM_REPORT_WORDS + i] = btok[i];
+	if (threadIdx.x == 0) {
+		out[0] = st->err;
+		out[1] = bad;
+		out[2] = st->tok;
+	}
+}
+
 /* kvcache_rotate's moves: dst[s * slab + i] = src[s * slab + i] */
 __global__ void k_lm_copy_rows(const float *__restrict__ src, float *__restrict__ dst,
 			       size_t slab, size_t n)
@@ -1517,6 +1561,38 @@ extern "C" int lm_launch_pick_rows(const float *logits, int nseq, int V, const L
 extern "C" int lm_launch_step_end(LmState *st, void *stream)
 {
 	hipLaunchKernelGGL(k_lm_step_end, dim3(1), dim3(64), 0, (hipStream_t)stream, st);
+	return (int)hipGetLastError();
+}
+
+extern "C" int lm_launch_set_state(LmState *st, const LmState *from, int *prompt, const int *ids,
+				   int n, void *stream)
+{
+	LmSet a;
+	if (n < 0 || n > LM_SET_IDS)
+		return (int)hipErrorInvalidValue;
+	a.st[0] = from->step;
+	a.st[1] = from->n_prompt;
+	a.st[2] = from->pos;
+	a.st[3] = from->size;
+	a.n = n;
+	for (int i = 0; i < n; i++)
+		a.ids[i] = ids[i];
+	hipLaunchKernelGGL(k_lm_set_state, dim3(1), dim3(LM_SET_IDS), 0, (hipStream_t)stream, st, prompt,
+			   a);
+	return (int)hipGetLastError();
+}
+
+extern "C" int lm_launch_report(const LmState *st, const int *btok, int nseq,
+				const uint32_t *const *err, int layers, int *out, void *stream)
+{
+	LmReport a;
+	if (layers < 0 || layers > LM_REPORT_LAYERS)
+		return (int)hipErrorInvalidValue;
+	a.layers = layers;
+	for (int i = 0; i < layers; i++)
+		a.err[i] = err[i];
+	hipLaunchKernelGGL(k_lm_report, dim3(1), dim3(256), 0, (hipStream_t)stream, st, btok, nseq, a,
+			   out);
 	return (int)hipGetLastError();
 }
 

@@ -166,6 +166,14 @@ int moe_launch_combine(const float *ypart, const float *w, float *out, int T,
 
 int moe_launch_expf(const float *in, float *out, size_t n, void *stream);
 int moe_launch_copy(const void *src, void *dst, size_t bytes, void *stream);
+/* up to four copies of 4-byte words in one launch, either side in pinned host
+ * memory; entries of no words are skipped */
+typedef struct moe_seg {
+	const void *src;
+	void *dst;
+	size_t words;
+} moe_seg;
+int moe_launch_copy_segs(const moe_seg *segs, int n, void *stream);
 
 /* Grouped path (moe_prefill.hip): sort by expert + f16 MFMA GEMMs. */
 #define MOE_WEIGHT_SLACK 256 /* bytes readable past the last weight row */
@@ -214,6 +222,9 @@ int moe_ffn_dev_norm(struct hip_moe_layer *L, const float *d_h, const float *d_n
  * was captured at another count names freed buffers and must be dropped. */
 struct hip_moe_layer;
 unsigned moe_scratch_gen(const struct hip_moe_layer *L);
+/* *word: the decode kernel's error word in device memory (NULL: the layer has
+ * no scratch yet); 0 where hip_moe_status would look at more than that */
+int moe_err_word(const struct hip_moe_layer *L, const uint32_t **word);
 
 /* Record an error message for hip_moe_last_error (and print it). */
 void moe_set_error(const char *msg);

@@ -592,6 +592,19 @@ __global__ __launch_bounds__(256) void k_copy(const uint4 *__restrict__ src,
 		dst[i] = src[i];
 }
 
+/* up to four copies of words; grid (blocks, copies) */
+struct copy_segs {
+	moe_seg s[4];
+};
+
+__global__ __launch_bounds__(256) void k_copy_segs(copy_segs a)
+{
+	const moe_seg g = a.s[blockIdx.y];
+	for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < g.words;
+	     i += (size_t)gridDim.x * 256)
+		((u32 *)g.dst)[i] = ((const u32 *)g.src)[i];
+}
+
 /* ------------------------------------------------------------------ */
 /* launchers                                                           */
 /* ------------------------------------------------------------------ */
@@ -760,5 +773,25 @@ extern "C" int moe_launch_copy(const void *src, void *dst, size_t bytes, void *s
 	dim3 grid((unsigned)(blocks < 8192 ? blocks : 8192));
 	hipLaunchKernelGGL(k_copy, grid, dim3(256), 0, (hipStream_t)stream, (const uint4 *)src,
 			   (uint4 *)dst, n);
+	return (int)hipGetLastError();
+}
+
+extern "C" int moe_launch_copy_segs(const moe_seg *segs, int n, void *stream)
+{
+	copy_segs a = {};
+	size_t most = 0;
+	int k = 0;
+	if (n < 0 || n > 4)
+		return (int)hipErrorInvalidValue;
+	for (int i = 0; i < n; i++)
+		if (segs[i].words) {
+			a.s[k++] = segs[i];
+			most = segs[i].words > most ? segs[i].words : most;
+		}
+	if (!k)
+		return 0;
+	const size_t blocks = (most + 255) / 256;
+	hipLaunchKernelGGL(k_copy_segs, dim3((unsigned)(blocks < 256 ? blocks : 256), k), dim3(256), 0,
+			   (hipStream_t)stream, a);
 	return (int)hipGetLastError();
 }
