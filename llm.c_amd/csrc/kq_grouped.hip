@@ -36,9 +36,9 @@
  * of vector_avx2.h:126-132 joins the eight tiles at the end.
  *
  * Measured (Q4_K gate/up, Q6_K down): 2048 x 1024, 64 experts top-8, 301
- * tokens: 3471 -> 291 us a layer against a workgroup per pair and 32 rows
- * (gate/up 930 -> 91, down 2608 -> 202 us); 4096 x 14336, 8 top-2, 200
- * tokens: 15762 -> 1018 us (6361 -> 291, 9176 -> 738).
+ * tokens: 3471 -> 280 us a layer against a workgroup per pair and 32 rows
+ * (gate/up 930 -> 91, down 2608 -> 187 us); 4096 x 14336, 8 top-2, 200
+ * tokens: 15762 -> 994 us (6361 -> 291, 9176 -> 700).
  */
 #include "kq_device.h"
 #include "moe_internal.h"
@@ -214,6 +214,9 @@ __device__ static inline void km_mins(const kmw<5> &, const uint8_t *, int, int,
 {
 }
 
+/* Both run in steps of two MFMAs, the next step's operands (LDS reads and
+ * unpacking) beside them: left to itself the scheduler reads every operand
+ * first and spills, or each right before its MFMA and waits for it. */
 template <int LR>
 __device__ static inline void km_sums(const kmw<3> &w, const uint8_t *sa, int m, int h,
 				      floatx16 &S1, floatx16 &S2)
@@ -222,28 +225,37 @@ __device__ static inline void km_sums(const kmw<3> &w, const uint8_t *sa, int m,
 	const u32 sc_lo = s0 & 0x3f3f3f3fu;
 	const u32 sc_hi = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
 	const floatx16 z = {};
-	S1 = z;
-	S2 = z;
-#pragma unroll
-	for (int j = 0; j < 4; j++) {
+	half8_t a[2][2], o[2][2]; /* [step & 1][low, high nibbles] */
+	auto operands = [&](int t) {
+		const int j = t / 2, u = t % 2;
 		const u32 sw = j < 2 ? sc_lo : sc_hi;
-		const _Float16 a = (_Float16)(float)((sw >> (16 * (j & 1))) & 0xff);
-		const _Float16 b = (_Float16)(float)((sw >> (16 * (j & 1) + 8)) & 0xff);
-		const _Float16 ao = (_Float16)-1024.0f * a, bs = (_Float16)0.0625f * b,
-			       bo = (_Float16)-64.0f * b;
-		const half2_t a2 = {a, a}, ao2 = {ao, ao}, b2 = {bs, bs}, bo2 = {bo, bo};
+		const _Float16 c = (_Float16)(float)((sw >> (16 * (j & 1))) & 0xff);
+		const _Float16 d = (_Float16)(float)((sw >> (16 * (j & 1) + 8)) & 0xff);
+		const _Float16 co = (_Float16)-1024.0f * c, ds = (_Float16)0.0625f * d,
+			       dof = (_Float16)-64.0f * d;
+		const half2_t c2 = {c, c}, co2 = {co, co}, d2 = {ds, ds}, do2 = {dof, dof};
+		a[t & 1][0] = km_a<LR>(sa, ((4 * j + u) * 2) + h, m);
+		a[t & 1][1] = km_a<LR>(sa, ((4 * j + 2 + u) * 2) + h, m);
+		const u32 x = w.dw(j, 2 * u), y = w.dw(j, 2 * u + 1);
+		o[t & 1][0] = km_op(x, y, 0x000f000fu, c2, co2);
+		o[t & 1][1] = km_op(x, y, 0x00f000f0u, d2, do2);
+	};
+	operands(0);
+	__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-		for (int u = 0; u < 2; u++) {
-			const u32 x = w.dw(j, 2 * u), y = w.dw(j, 2 * u + 1);
-			const half8_t lo = km_op(x, y, 0x000f000fu, a2, ao2);
-			const half8_t hi = km_op(x, y, 0x00f000f0u, b2, bo2);
-			const half8_t al = km_a<LR>(sa, ((4 * j + u) * 2) + h, m);
-			const half8_t ah = km_a<LR>(sa, ((4 * j + 2 + u) * 2) + h, m);
-			floatx16 &S = j < 2 ? S1 : S2;
-			S = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, lo, S, 0, 0, 0);
-			S = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, hi, S, 0, 0, 0);
+	for (int t = 0; t < 8; t++) {
+		if (t + 1 < 8)
+			operands(t + 1);
+		floatx16 &S = t < 4 ? S1 : S2;
+		S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t & 1][0], o[t & 1][0], t & 3 ? S : z, 0, 0,
+							   0);
+		S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t & 1][1], o[t & 1][1], S, 0, 0, 0);
+		__builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+		for (int i = 0; i < 2; i++) {
+			__builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+			__builtin_amdgcn_sched_group_barrier(0x2, 14, 0);
 		}
-		/* left to itself the scheduler reads every operand first and spills */
 		__builtin_amdgcn_sched_barrier(0);
 	}
 }
@@ -253,34 +265,41 @@ __device__ static inline void km_sums(const kmw<5> &w, const uint8_t *sa, int m,
 				      floatx16 &S1, floatx16 &S2)
 {
 	const floatx16 z = {};
-	S1 = z;
-	S2 = z;
+	half8_t a[2], o[2][2]; /* [step & 1][sl, sh] */
+	auto operands = [&](int t) {
+		const int i = t / 2, u = t % 2, c = i / 4, g = i % 4;
+		/* values 32 i ..; sub-block 2 i + h */
+		const int sc = (int)(int8_t)((w.sc[i / 2] >> (16 * (i & 1) + 8 * h)) & 0xff);
+		const _Float16 sl = (_Float16)(float)(sc & 15), sh = (_Float16)(float)(sc >> 4);
+		const _Float16 slo = (_Float16)-1056.0f * sl, sho = (_Float16)-1056.0f * sh;
+		const half2_t sl2 = {sl, sl}, slo2 = {slo, slo}, sh2 = {sh, sh}, sho2 = {sho, sho};
+		u32 v[2];
 #pragma unroll
-	for (int c = 0; c < 2; c++)
-#pragma unroll
-		for (int g = 0; g < 4; g++) {
-			const int i = 4 * c + g; /* values 32 i ..; sub-block 2 i + h */
-			const int sc = (int)(int8_t)((w.sc[i / 2] >> (16 * (i & 1) + 8 * h)) & 0xff);
-			const _Float16 sl = (_Float16)(float)(sc & 15), sh = (_Float16)(float)(sc >> 4);
-			const _Float16 slo = (_Float16)-1056.0f * sl, sho = (_Float16)-1056.0f * sh;
-			const half2_t sl2 = {sl, sl}, slo2 = {slo, slo}, sh2 = {sh, sh}, sho2 = {sho, sho};
-#pragma unroll
-			for (int u = 0; u < 2; u++) {
-				u32 v[2];
-#pragma unroll
-				for (int k = 0; k < 2; k++) {
-					const u32 q = w.ql[2 * c + (g & 1)][2 * u + k];
-					const u32 lo = g < 2 ? q & 0x0f0f0f0fu : (q >> 4) & 0x0f0f0f0fu;
-					v[k] = lo | (((w.qh[c][2 * u + k] >> (2 * g)) & 0x03030303u) << 4);
-				}
-				const half8_t a = km_a<LR>(sa, ((2 * i + u) * 2) + h, m);
-				S1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-					a, km_op(v[0], v[1], 0x00ff00ffu, sl2, slo2), S1, 0, 0, 0);
-				S2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-					a, km_op(v[0], v[1], 0x00ff00ffu, sh2, sho2), S2, 0, 0, 0);
-			}
-			__builtin_amdgcn_sched_barrier(0);
+		for (int k = 0; k < 2; k++) {
+			const u32 q = w.ql[2 * c + (g & 1)][2 * u + k];
+			const u32 lo = g < 2 ? q & 0x0f0f0f0fu : (q >> 4) & 0x0f0f0f0fu;
+			v[k] = lo | (((w.qh[c][2 * u + k] >> (2 * g)) & 0x03030303u) << 4);
 		}
+		a[t & 1] = km_a<LR>(sa, ((2 * i + u) * 2) + h, m);
+		o[t & 1][0] = km_op(v[0], v[1], 0x00ff00ffu, sl2, slo2);
+		o[t & 1][1] = km_op(v[0], v[1], 0x00ff00ffu, sh2, sho2);
+	};
+	operands(0);
+	__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+	for (int t = 0; t < 16; t++) {
+		if (t + 1 < 16)
+			operands(t + 1);
+		S1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t & 1], o[t & 1][0], t ? S1 : z, 0, 0, 0);
+		S2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t & 1], o[t & 1][1], t ? S2 : z, 0, 0, 0);
+		__builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+		for (int i = 0; i < 2; i++) {
+			__builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+			__builtin_amdgcn_sched_group_barrier(0x2, 16, 0);
+		}
+		__builtin_amdgcn_sched_barrier(0);
+	}
 }
 
 /* the fp32 step of one super-block: acc = fma(yd * d, sumi, acc) */
@@ -651,11 +670,18 @@ template <> struct kdw<5> {
 
 /*
  * Bound: the fp32 matrix rate (157 TFLOP/s; the reference's order leaves no
- * faster unit): 4096 x 14336, 400 pairs, 47 GFLOP = 300 us without padding.
+ * faster unit): 4096 x 14336, 400 pairs, 47 GFLOP = 300 us without padding;
+ * about 38 cycles a 16x16x4 instruction measured where 32 are nominal, and the
+ * unpacking's VALU cycles add to them.
  * Eight chains of 16 x 16 accumulators per half tile and wave keep the
  * matrix core's latency covered; a wave unpacks its own 16 rows' weights
  * (26 VALU instructions per 8 MFMAs of a half tile), and the rows' h comes
- * through LDS, shared by the four waves (two buffers of a super-block).
+ * through LDS, shared by the four waves (two buffers of a super-block).  The
+ * loads of the next super-block go out at its top and a step's operands are
+ * made one step ahead, both held there by hand (the compiler put each right
+ * before its use): 831 -> 786 us at 400 pairs of 4096 x 14336, 202 -> 187 at
+ * 2408 of 2048 x 1024 under a profiler.  Weights two super-blocks ahead
+ * measured 7% slower (the copies between register sets wait for the loads).
  */
 /* NS 16-row halves of the tile in use.  Wave w: down rows cb * 64 + 16 w ..
  * + 15; MFMA step (s, c): element 32 s + 8 k + c of chain c, k = lane / 16 */
@@ -702,23 +728,38 @@ __device__ static inline void kd_tile(const uint8_t *__restrict__ base, int nb,
 		const int nx = min(sb + 1, nb - 1);
 		fetch(nx);
 		wn.load(row + (size_t)nx * BY, g);
+		/* here, not next to their use a super-block later, where the
+		 * compiler would put them */
+		__builtin_amdgcn_sched_barrier(0);
 		const float *sh = s_h + (size_t)(sb & 1) * (KM_ROWS * KW_HS) + m * KW_HS + 8 * g;
-#pragma unroll
-		for (int s = 0; s < 8; s++) {
-			float v[8];
-			w.values(s, g, v);
-			floatx4 a[NS][2];
+		float v[2][8];
+		floatx4 a[2][NS][2];
+		auto operands = [&](int s) {
 #pragma unroll
 			for (int n = 0; n < NS; n++) {
-				a[n][0] = *(const floatx4 *)(sh + n * 16 * KW_HS + 32 * s);
-				a[n][1] = *(const floatx4 *)(sh + n * 16 * KW_HS + 32 * s + 4);
+				a[s & 1][n][0] = *(const floatx4 *)(sh + n * 16 * KW_HS + 32 * s);
+				a[s & 1][n][1] = *(const floatx4 *)(sh + n * 16 * KW_HS + 32 * s + 4);
 			}
+			w.values(s, g, v[s & 1]);
+		};
+		operands(0);
+#pragma unroll
+		for (int s = 0; s < 8; s++) { /* the next operands beside this step's MFMAs */
+			if (s + 1 < 8)
+				operands(s + 1);
 #pragma unroll
 			for (int c = 0; c < 8; c++)
 #pragma unroll
 				for (int n = 0; n < NS; n++)
 					acc[c][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-						a[n][c / 4][c % 4], v[c], acc[c][n], 0, 0, 0);
+						a[s & 1][n][c / 4][c % 4], v[s & 1][c], acc[c][n], 0, 0, 0);
+			__builtin_amdgcn_sched_group_barrier(0x100, 2 * NS, 0);
+#pragma unroll
+			for (int i = 0; i < 8 * NS; i++) {
+				__builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+				__builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+			}
+			__builtin_amdgcn_sched_barrier(0);
 		}
 		stage((sb + 1) & 1);
 		w = wn;
