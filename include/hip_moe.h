@@ -292,7 +292,7 @@ hip_moe_qmat *hip_moe_qmat_upload(const void *qdata, int wtype, size_t N, size_t
  * dot_q4_K_q8_K / dot_q6_K_q8_K, quant_avx2.h:8-209): there every output
  * equals the reference's bit for bit (the integer sums are exact and the
  * fp32 steps are the reference's, in its order), several tokens (from
- * 7 to 14 on) on the matrix cores.  Returns 1 on success, 0 if not applicable.
+ * 6 to 10 on) on the matrix cores.  Returns 1 on success, 0 if not applicable.
  */
 int hip_moe_qmat_mul(hip_moe_qmat *W, const float *x, size_t T, const float *add,
                      size_t add_len, float *out);

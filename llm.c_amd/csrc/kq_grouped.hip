@@ -38,7 +38,7 @@
  * Measured (Q4_K gate/up, Q6_K down): 2048 x 1024, 64 experts top-8, 301
  * tokens: 3471 -> 280 us a layer against a workgroup per pair and 32 rows
  * (gate/up 930 -> 91, down 2608 -> 187 us); 4096 x 14336, 8 top-2, 200
- * tokens: 15762 -> 994 us (6361 -> 291, 9176 -> 700).
+ * tokens: 15762 -> 994 us (6361 -> 291, 9176 -> about 690).
  */
 #include "kq_device.h"
 #include "moe_internal.h"
@@ -447,6 +447,23 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 /* the dense product                                                    */
 /* ------------------------------------------------------------------ */
 
+/* the value of lane ^ 1, of lane ^ 2, of the mirrored lane among eight: VALU
+ * moves, where a shuffle goes through LDS (whose round trips, one after the
+ * other, took most of kq_stage's time) */
+template <int CTRL> __device__ static inline int km_dpp(int v)
+{
+	return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+
+template <int CTRL> __device__ static inline float km_dpp(float v)
+{
+	return __builtin_bit_cast(float, km_dpp<CTRL>(__builtin_bit_cast(int, v)));
+}
+
+#define KM_X1 0xb1  /* quad_perm 1 0 3 2 */
+#define KM_X2 0x4e  /* quad_perm 2 3 0 1 */
+#define KM_M8 0x141 /* row_half_mirror */
+
 /*
  * quantize_row_q8 (quant.c:627-654) of one super-block of a tile's 32 rows
  * into operand chunks at sa and scales at yd, by 256 threads: eight a row,
@@ -464,11 +481,12 @@ __device__ static inline void kq_stage(const float4 (&v)[8], uint8_t *sa, float 
 		hi = fmaxf(fmaxf(fmaxf(hi, v[j].x), fmaxf(v[j].y, v[j].z)), v[j].w);
 		lo = fminf(fminf(fminf(lo, v[j].x), fminf(v[j].y, v[j].z)), v[j].w);
 	}
-#pragma unroll
-	for (int off = 1; off < 8; off <<= 1) {
-		hi = fmaxf(hi, __shfl_xor(hi, off, WAVE));
-		lo = fminf(lo, __shfl_xor(lo, off, WAVE));
-	}
+	hi = fmaxf(hi, km_dpp<KM_X1>(hi));
+	lo = fminf(lo, km_dpp<KM_X1>(lo));
+	hi = fmaxf(hi, km_dpp<KM_X2>(hi));
+	lo = fminf(lo, km_dpp<KM_X2>(lo));
+	hi = fmaxf(hi, km_dpp<KM_M8>(hi));
+	lo = fminf(lo, km_dpp<KM_M8>(lo));
 	float bv = hi > -lo ? hi : lo;
 	if (hi == -lo && hi > 0.0f) { /* the eight threads of a row agree */
 		int key = 0x7fffffff;
@@ -502,8 +520,8 @@ __device__ static inline void kq_stage(const float4 (&v)[8], uint8_t *sa, float 
 			o[k == 1 ? 2 : k == 2 ? 1 : k] = (_Float16)(float)(int8_t)(q & 0xff);
 		}
 		*(half4_t *)(sa + ((2 * j + u) * 2 + h) * LR + row * 16 + (i & 1) * 8) = o;
-		s += __shfl_xor(s, 1, WAVE);
-		s += __shfl_xor(s, 2, WAVE);
+		s += km_dpp<KM_X1>(s);
+		s += km_dpp<KM_X2>(s);
 		/* sum i / 4 + 2 j of 16 values, finite in f16 as in k_kq_rec */
 		if ((i & 3) == 0)
 			*(_Float16 *)(sa + (32 + (j >> 2)) * LR + row * 16 + 2 * ((h + 2 * j) & 7)) =
@@ -513,24 +531,26 @@ __device__ static inline void kq_stage(const float4 (&v)[8], uint8_t *sa, float 
 		yd[row] = zero ? 0.0f : 1.0f / iscale;
 }
 
-#define KD_WAVES 4
+#define KD_WAVES 4 /* of a workgroup's eight: the ones that multiply */
 
 /*
  * out = add + x . W^T for T tokens: a workgroup takes a tile of 32 tokens and
  * 128 columns, as k_kq_mm takes one matrix, but quantizes its tokens itself
  * into the LDS buffer the next super-block is read from: a call then holds no
- * scratch memory, so calls on one matrix may overlap and be captured.  The
- * quantization is done again for every 128 columns; it costs about as many
- * VALU cycles as the operands of one wave's 32 columns.
+ * scratch memory, so calls on one matrix may overlap and be captured.  Four
+ * waves multiply, four quantize the next super-block meanwhile (one of each
+ * on every SIMD): the quantization is done again for every 128 columns and
+ * costs about as much as the operands of one wave's 32 columns.
  *
- * Bound: the VALU, in series with the MFMAs where a call has fewer than two
- * workgroups per CU.  4096 x 4096 Q4_K: 77 tokens 384 -> 47 us, 333 tokens
- * 1771 -> 71 us against the per-token product (whose groups of tokens re-read
- * and re-unpack every weight); Q6_K 390 -> 78 and 1772 -> 115 us; 4096 x 14336
- * Q4_K, 77 tokens: 2132 -> 154 us.
+ * Bound: the VALU, which the MFMAs' cycles add to where they share a SIMD.
+ * 4096 x 4096 Q4_K: 77 tokens 384 -> 42 us, 333 tokens 1771 -> 70 us against
+ * the per-token product (whose groups of tokens re-read and re-unpack every
+ * weight); Q6_K 390 -> 55 and 1772 -> 96 us; 4096 x 14336 Q4_K, 77 tokens:
+ * 2132 -> 140 us.  With every wave quantizing and then multiplying: 47, 71,
+ * 78, 115 and 154 us.
  */
 template <int WT>
-__global__ __launch_bounds__(KD_WAVES * WAVE, 2) void k_kq_dense(
+__global__ __launch_bounds__(2 * KD_WAVES * WAVE, 4) void k_kq_dense(
 	const uint8_t *__restrict__ W, const float *__restrict__ x, int T, int K, int N,
 	const float *__restrict__ add, int add_rows, float *__restrict__ out)
 {
@@ -547,34 +567,50 @@ __global__ __launch_bounds__(KD_WAVES * WAVE, 2) void k_kq_dense(
 	const int tile = item % ntiles, col = item / ntiles * (KD_WAVES * 32) + wave * 32 + m;
 	/* columns past N repeat the last one, rows past T the last token (never stored) */
 	const uint8_t *wp = W + (size_t)min(col, N - 1) * nb * BY;
-	const int row = tid >> 3, i = tid & 7;
-	const float4 *xp = (const float4 *)(x + (size_t)min(tile * KM_ROWS + row, T - 1) * K) + i;
-	float4 v[8];
+	if (wave >= KD_WAVES) { /* quantize: eight threads a token */
+		const int pt = tid - KD_WAVES * WAVE, row = pt >> 3, i = pt & 7;
+		const float4 *xp =
+			(const float4 *)(x + (size_t)min(tile * KM_ROWS + row, T - 1) * K) + i;
+		float4 v[8];
+		auto fetch = [&](int sb) {
+#pragma unroll
+			for (int j = 0; j < 8; j++)
+				v[j] = xp[(size_t)min(sb, nb - 1) * 64 + 8 * j];
+		};
+		fetch(0);
+		kq_stage(v, s_a[0], s_yd[0], row, i);
+		fetch(1);
+		for (int sb = 0; sb < nb; sb++) {
+			__syncthreads(); /* buffer sb & 1 is whole, the other one is free */
+			if (sb + 1 < nb)
+				kq_stage(v, s_a[(sb & 1) ^ 1], s_yd[(sb & 1) ^ 1], row, i);
+			fetch(sb + 2);
+		}
+		return;
+	}
 	kmw<WT> w;
 	floatx16 acc = {}, accm = {};
-#pragma unroll
-	for (int j = 0; j < 8; j++)
-		v[j] = xp[8 * j];
 	w.load(wp, h);
-	kq_stage(v, s_a[0], s_yd[0], row, i);
 	for (int sb = 0; sb < nb; sb++) {
-		const int nx = min(sb + 1, nb - 1), b = sb & 1;
-		__syncthreads(); /* buffer b is whole, the other one is free */
-#pragma unroll
-		for (int j = 0; j < 8; j++)
-			v[j] = xp[(size_t)nx * 64 + 8 * j];
+		const int b = sb & 1;
+		__syncthreads(); /* the other waves' one */
+		/* the next super-block's; Q6_K's only once the sums' operands are
+		 * done with (128 registers hold two workgroups a CU) */
+		kmw<WT> wn;
+		const uint8_t *next = wp + (size_t)min(sb + 1, nb - 1) * BY;
+		if (WT == 3)
+			wn.load(next, h);
+		__builtin_amdgcn_sched_barrier(0);
 		const floatx4 *yd = (const floatx4 *)(s_yd[b] + 4 * h);
 		floatx16 S1, S2;
 		km_mins<LR>(w, s_a[b], m, h, yd, accm);
 		__builtin_amdgcn_sched_barrier(0);
 		km_sums<LR>(w, s_a[b], m, h, S1, S2);
+		if (WT != 3)
+			wn.load(next, h);
+		__builtin_amdgcn_sched_barrier(0);
 		km_step(w, S1, S2, yd, acc);
-		__builtin_amdgcn_sched_barrier(0);
-		/* the next super-block's, into the registers just read */
-		w.load(wp + (size_t)nx * BY, h);
-		__builtin_amdgcn_sched_barrier(0);
-		if (sb + 1 < nb)
-			kq_stage(v, s_a[b ^ 1], s_yd[b ^ 1], row, i);
+		w = wn;
 	}
 	if (col >= N)
 		return;
@@ -864,18 +900,16 @@ extern "C" int moe_launch_kq_grouped(int gt, int dt, const uint8_t *gate, const 
 }
 
 /* A tile costs the same for 1 and for 32 tokens, the per-token product grows
- * with T.  Where they cross, per-token / tile in us: Q4_K 4096 x 4096 T = 8
- * 45.0 / 45.5, T = 12 63.6 / 45.8; 2048 x 2048 T = 8 23.7 / 24.5, T = 12
- * 35.0 / 24.9; Q6_K 4096 x 4096 T = 12 65.3 / 76.5, T = 16 84.0 / 76.4; 2048 x
- * 2048 T = 12 38.6 / 39.3, T = 16 49.0 / 39.3.  Matrices whose 128-row blocks
- * fill half the chip or more cross earlier: Q4_K 50304 x 2048 T = 7 46.5 /
- * 38, 32000 x 4096 T = 7 90 / 50; Q6_K T = 8 60.1 / 59 and 93 / 87, T = 9 78 /
- * 59 and 119 / 87 */
+ * with T.  Where they cross, per-token / tile in us: Q4_K 4096 x 4096 T = 7
+ * 40.6 / 40.3, T = 8 45.7 / 40.3; 2048 x 2048 T = 7 21.3 / 22.1, T = 8 23.6 /
+ * 22.1; Q6_K 4096 x 4096 T = 9 51.3 / 53.0, T = 10 55.7 / 53.0; 2048 x 2048 T =
+ * 9 30.9 / 28.0.  Matrices whose 128-row blocks fill half the chip or more
+ * cross earlier: Q4_K 50304 x 2048 T = 6 41.9 / 36.3; Q6_K T = 7 55.0 / 49.9 */
 extern "C" int moe_kq_dense_better(int wtype, size_t N, size_t T)
 {
 	if (N >= 16384)
-		return T >= (wtype == 3 ? 7 : 9);
-	return T >= (wtype == 3 ? 9 : 14);
+		return T >= (wtype == 3 ? 6 : 7);
+	return T >= (wtype == 3 ? 8 : 10);
 }
 
 extern "C" int moe_launch_kq_dense(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
@@ -885,7 +919,7 @@ extern "C" int moe_launch_kq_dense(int wtype, const uint8_t *W, int N, int K, co
 				((N + KD_WAVES * 32 - 1) / (KD_WAVES * 32));
 	if ((wtype != 3 && wtype != 5) || N < 1 || T < 1 || K < 256 || K % 256 || items > 0x7fffff00ll)
 		return (int)hipErrorInvalidValue;
-	const dim3 grid((unsigned)((items + 7) / 8 * 8)), blk(KD_WAVES * WAVE);
+	const dim3 grid((unsigned)((items + 7) / 8 * 8)), blk(2 * KD_WAVES * WAVE);
 	hipStream_t s = (hipStream_t)stream;
 	if (wtype == 3)
 		hipLaunchKernelGGL(k_kq_dense<3>, grid, blk, 0, s, W, x, T, K, N, add, add_rows, out);
