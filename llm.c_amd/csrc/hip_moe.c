@@ -1245,7 +1245,7 @@ int hip_moe_qmat_mul_dev(const hip_moe_qmat *W, const float *d_x, size_t T,
 	} else if (T > 1 && W->qmm &&
 		   (T > W->split_T || moe_qmm_tile_better((int)W->N, (int)T))) {
 		/* several tokens: on the matrix cores, at fp32 accuracy; in tiles of
-		 * 64 tokens where those are faster or the split buffer holds fewer */
+		 * tokens where those are faster or the split buffer holds fewer */
 		LCHK(moe_launch_qmm_tile(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 					 add_len == T * W->N, d_out, s), "qmm_tile");
 	} else if (T > 1 && W->qmm) {

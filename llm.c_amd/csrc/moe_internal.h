@@ -75,7 +75,7 @@ int moe_qmm_supported(int wtype, int K);
 size_t moe_qmm_work_bytes(int T, int N, int K);
 int moe_launch_qmm(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
                    const float *add, int add_rows, float *out, void *work, void *stream);
-/* the same product in tiles of 64 tokens, without scratch memory; K a
+/* the same product in tiles of 32 or 64 tokens, without scratch memory; K a
  * multiple of 128; moe_qmm_tile_better: whether it is the faster of the two */
 int moe_qmm_tile_better(int N, int T);
 int moe_launch_qmm_tile(int wtype, const uint8_t *W, int N, int K, const float *x, int T,

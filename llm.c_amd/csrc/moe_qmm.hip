@@ -42,7 +42,7 @@
  * launches at 16 tokens x 6144 x 4096 Q4_0: the last arrivals' polls sit
  * in series behind the slowest stretch.)
  *
- * Many tokens, or very many rows, take k_qmm_tile below: tiles of 64 tokens
+ * Many tokens, or very many rows, take k_qmm_tile below: tiles of 32 or 64 tokens
  * over the whole of K, the tokens scaled per 128 columns.
  *
  * Bound of k_qmm: HBM for a few tokens (the weights are read once per token tile;
@@ -292,23 +292,26 @@ __global__ __launch_bounds__(256) void k_qmm_reduce(const float *__restrict__ pa
 /* the product of many tokens                                              */
 /* ---------------------------------------------------------------------- */
 
-#define QT_TOK 64                   /* tokens of a tile */
 #define QT_WAVES 8
-#define QT_COLS 128                 /* columns of K per stage: 4 blocks */
-#define QT_CHUNK (QT_TOK * 16 + 64) /* LDS bytes of one 16-byte chunk of every token; the
-				     * padding starts a wave's four chunks 16 banks apart */
-#define QT_XB (32 * QT_CHUNK)       /* a stage's tokens: 16 chunks of hi, 16 of lo */
+#define QT_COLS 128 /* columns of K per stage: 4 blocks */
 
-/* geometry of NW column waves: rows, bytes of a row's stage, stage bytes */
-template <int WT, int NW> struct qt_geo {
+/* geometry of TM 32-token groups and NW column waves: rows, bytes of a row's
+ * stage, stage bytes */
+template <int WT, int NW, int TM> struct qt_geo {
+	static constexpr int TOK = 32 * TM; /* tokens of a tile */
+	/* LDS bytes of one 16-byte chunk of every token; the padding starts a
+	 * wave's four chunks 16 banks apart */
+	static constexpr int CHUNK = TOK * 16 + 64;
+	static constexpr int XB = 32 * CHUNK;           /* a stage's tokens: 16 chunks of hi, 16 of lo */
+	static constexpr int TPR = QT_WAVES * WAVE / TOK; /* threads that stage a token */
 	static constexpr int BB = WT == 1 ? 34 : 18;
 	static constexpr int NR = 32 * NW;
 	static constexpr int RB = 4 * BB, DW = RB / 4;
 	/* dwords a thread loads; the last ones may repeat the last row past the tile */
 	static constexpr int J = (NR * DW + QT_WAVES * WAVE - 1) / (QT_WAVES * WAVE);
 	static constexpr int WB = J * QT_WAVES * WAVE * 4;
-	static constexpr int SB = QT_XB + WB; /* one stage */
-	static constexpr int LDS = 2 * SB + 2 * QT_TOK * 4;
+	static constexpr int SB = XB + WB; /* one stage */
+	static constexpr int LDS = 2 * SB + 2 * TOK * 4;
 };
 
 /* a lane's share of block b (parity ODD) of its row's stage in LDS: raw
@@ -388,32 +391,32 @@ template <int ODD> struct qt_blk<1, ODD> {
 };
 
 /*
- * NBK blocks of a stage for one wave: 64 tokens x 32 rows, each block's sums
+ * NBK blocks of a stage for one wave: 32 TM tokens x 32 rows, each block's sums
  * scaled by the row's block scale, their total by the tokens' scales into
  * tot.  Software-pipelined by hand in steps of half a block (its hi, then its
- * lo operands): a step's four MFMAs run beside the next step's LDS reads, the
+ * lo operands): a step's MFMAs run beside the next step's LDS reads, the
  * fp32 steps of the block before and the unpacking of the block after (left
  * to itself the compiler reads each operand right before its MFMA and waits
  * out the LDS latency every time).
  */
-template <int WT, int NBK>
+template <int WT, int NBK, int TM>
 __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, const float *sts, int r,
-					int h, floatx16 (&tot)[2])
+					int h, floatx16 (&tot)[TM])
 {
-	constexpr int BB = qt_geo<WT, 8>::BB;
+	constexpr int BB = qt_geo<WT, 8, TM>::BB, CH = qt_geo<WT, 8, TM>::CHUNK;
 	qt_blk<WT, 0> we;
 	qt_blk<WT, 1> wo;
-	half8_t k[2][2], a[2][2][2]; /* k: [block & 1][kh]; a: [step & 1][kh][t] */
-	floatx16 s[2][2], acc[2];
+	half8_t k[2][2], a[2][2][TM]; /* k: [block & 1][kh]; a: [step & 1][kh][t] */
+	floatx16 s[2][TM], acc[TM];
 	float d[2];
 	auto reada = [&](int step) {
 		const int b = step / 2, p = step % 2;
 #pragma unroll
 		for (int kh = 0; kh < 2; kh++)
 #pragma unroll
-			for (int t = 0; t < 2; t++)
+			for (int t = 0; t < TM; t++)
 				a[step & 1][kh][t] = *(const half8_t *)(
-					sx + (16 * p + 4 * b + 2 * kh + h) * QT_CHUNK + (32 * t + r) * 16);
+					sx + (16 * p + 4 * b + 2 * kh + h) * CH + (32 * t + r) * 16);
 	};
 	we.load(row, h);
 	wo.load(row + BB, h);
@@ -441,7 +444,7 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 #pragma unroll
 		for (int kh = 0; kh < 2; kh++)
 #pragma unroll
-			for (int t = 0; t < 2; t++) {
+			for (int t = 0; t < TM; t++) {
 				const floatx16 z = {};
 				s[f][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
 					a[step & 1][kh][t], k[f][kh], p == 0 && kh == 0 ? z : s[f][t], 0, 0, 0);
@@ -449,7 +452,7 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 		if (b > 0 && p == 0) { /* the block before (the next step's unpacking replaces d) */
 			const float e = d[f ^ 1];
 #pragma unroll
-			for (int t = 0; t < 2; t++)
+			for (int t = 0; t < TM; t++)
 #pragma unroll
 				for (int j = 0; j < 16; j++)
 					acc[t][j] = b == 1 ? e * s[f ^ 1][t][j]
@@ -457,7 +460,7 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 		}
 		__builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-		for (int i = 0; i < 4; i++) {
+		for (int i = 0; i < 2 * TM; i++) {
 			__builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
 			__builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
 		}
@@ -466,7 +469,7 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 	const floatx4 *ts = (const floatx4 *)(sts + 4 * h);
 	constexpr int f = (NBK - 1) & 1;
 #pragma unroll
-	for (int t = 0; t < 2; t++)
+	for (int t = 0; t < TM; t++)
 #pragma unroll
 		for (int j = 0; j < 16; j++)
 			tot[t][j] = __builtin_fmaf(ts[8 * t + 2 * (j / 4)][j % 4],
@@ -474,26 +477,31 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 }
 
 /*
- * A token's 128 columns of a stage, held by eight threads (thread i: the
- * float4s i of the four blocks), scaled by one power of two (the largest
+ * A token's 128 columns of a stage, held by TPR = 8 or 16 threads (thread i:
+ * the float4s i, i + TPR, ...), scaled by one power of two (the largest
  * magnitude into [2^13, 2^14)) and split into hi and lo.
  */
-__device__ static inline void qt_stage(const float4 (&v)[4], uint8_t *sx, float *ts, int row, int i)
+template <int TPR, int CH>
+__device__ static inline void qt_stage(const float4 (&v)[32 / TPR], uint8_t *sx, float *ts, int row, int i)
 {
 	typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 	float m = 0.0f;
 #pragma unroll
-	for (int j = 0; j < 4; j++) {
+	for (int j = 0; j < 32 / TPR; j++) {
 		m = fmaxf(fmaxf(m, fabsf(v[j].x)), fabsf(v[j].y));
 		m = fmaxf(fmaxf(m, fabsf(v[j].z)), fabsf(v[j].w));
 	}
-	/* the eight threads' maximum: lanes ^ 1, ^ 2, then the other four mirrored */
+	/* the threads' maximum: lanes ^ 1, ^ 2, the other four mirrored, the other
+	 * eight mirrored */
 	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0xb1,
 									0xf, 0xf, true)));
 	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x4e,
 									0xf, 0xf, true)));
 	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x141,
 									0xf, 0xf, true)));
+	if constexpr (TPR == 16)
+		m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(
+						   __builtin_bit_cast(int, m), 0x140, 0xf, 0xf, true)));
 	int sh = 0;
 	if (m > 0.0f) { /* 13 - exponent; the largest scale a float holds below that */
 		sh = 140 - (int)((__builtin_bit_cast(u32, m) >> 23) & 0xffu);
@@ -501,7 +509,7 @@ __device__ static inline void qt_stage(const float4 (&v)[4], uint8_t *sx, float 
 	}
 	const float s = __builtin_bit_cast(float, (u32)(sh + 127) << 23);
 #pragma unroll
-	for (int j = 0; j < 4; j++) {
+	for (int j = 0; j < 32 / TPR; j++) {
 		/* element order 0, 2, 1, 3: a weight operand's */
 		const float y[4] = {v[j].x * s, v[j].z * s, v[j].y * s, v[j].w * s};
 		half4_t hi, lo;
@@ -510,16 +518,17 @@ __device__ static inline void qt_stage(const float4 (&v)[4], uint8_t *sx, float 
 			hi[k] = (_Float16)y[k];
 			lo[k] = (_Float16)(y[k] - (float)hi[k]);
 		}
-		uint8_t *o = sx + (4 * j + (i >> 1)) * QT_CHUNK + row * 16 + (i & 1) * 8;
+		const int f = i + TPR * j; /* of the token's 32 float4s: block f / 8 */
+		uint8_t *o = sx + (f >> 1) * CH + row * 16 + (f & 1) * 8;
 		*(half4_t *)o = hi;
-		*(half4_t *)(o + 16 * QT_CHUNK) = lo;
+		*(half4_t *)(o + 16 * CH) = lo;
 	}
 	if (i == 0)
 		ts[row] = __builtin_bit_cast(float, (u32)(127 - sh) << 23);
 }
 
 /*
- * out = add + x . W^T, a workgroup of eight waves per (64 tokens, 32 NW rows):
+ * out = add + x . W^T, a workgroup of eight waves per (32 TM tokens, 32 NW rows):
  * NW waves side by side on the rows, and 8 / NW groups of them on the blocks
  * of a stage (128 columns of K), whose sums are added at the end in group
  * order.  The raw weights of a stage come by LDS-DMA and the tokens through
@@ -528,34 +537,34 @@ __device__ static inline void qt_stage(const float4 (&v)[4], uint8_t *sx, float 
  * matrix may overlap and be captured.
  *
  * Bound: the VALU (the tokens' split, the unpacking, one fp32 step per block
- * and output) and the MFMAs, each about 2,500 cycles of a stage's 6,000, in a
- * single workgroup per CU (LDS).  Q4_0 6144 x 4096, 333 tokens: 926 -> 85 us
+ * and output) and the MFMAs, each about 2,500 cycles of a 64 x 256 stage's
+ * 6,000, in a single workgroup per CU (LDS); two 32 x 128 ones fit.  Q4_0 6144 x 4096, 333 tokens: 926 -> 85 us
  * (the per-token product, which takes the weights once per token), 1024
  * tokens against k_qmm 908 -> 184; 4096 x 4096, 1024 tokens 608 -> 101.  Tried:
  * 32 tokens x 64 rows a wave (half the operand reads, twice the unpacking)
  * 91 -> 101; splitting the tokens at opposite ends of a stage in a SIMD's two
  * waves 91 -> 96; without the hand-pipelined order 104.
  */
-template <int WT, int NW>
-__global__ __launch_bounds__(QT_WAVES * WAVE) void k_qmm_tile(
+template <int WT, int NW, int TM>
+__global__ __launch_bounds__(QT_WAVES * WAVE, TM == 1 ? 4 : 2) void k_qmm_tile(
 	const uint8_t *__restrict__ W, size_t rb, int N, int K, const float *__restrict__ x, int T,
 	const float *__restrict__ add, int add_rows, float *__restrict__ out)
 {
-	typedef qt_geo<WT, NW> G;
+	typedef qt_geo<WT, NW, TM> G;
 	constexpr int KG = QT_WAVES / NW, GB = 4 / KG; /* K groups; blocks of a stage each takes */
 	__shared__ __attribute__((aligned(16))) uint8_t qt_lds[G::LDS];
 	float *s_ts = (float *)(qt_lds + 2 * G::SB); /* [2][64] */
 	const int tid = threadIdx.x, lane = tid % WAVE;
 	const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
 	const int r = lane & 31, h = lane >> 5, wn = wave % NW, wk = wave / NW;
-	const int tiles = (T + QT_TOK - 1) / QT_TOK, cols = (N + G::NR - 1) / G::NR;
+	const int tiles = (T + G::TOK - 1) / G::TOK, cols = (N + G::NR - 1) / G::NR;
 	/* class id % 8 (an XCD) takes a contiguous run of items, a column block's
 	 * token tiles side by side: they share its weights in that L2 */
 	const int per = (tiles * cols + 7) / 8, item = ((int)blockIdx.x % 8) * per + (int)blockIdx.x / 8;
 	if ((int)blockIdx.x / 8 >= per || item >= tiles * cols)
 		return; /* the whole workgroup */
-	const int t0 = item % tiles * QT_TOK, n0 = item / tiles * G::NR;
-	const int row = tid >> 3, i = tid & 7;
+	const int t0 = item % tiles * G::TOK, n0 = item / tiles * G::NR;
+	const int row = tid / G::TPR, i = tid % G::TPR;
 	/* tokens past T repeat the last one, rows past N the last row (never stored) */
 	const float4 *xp = (const float4 *)(x + (size_t)min(t0 + row, T - 1) * K) + i;
 	const uint8_t *wb = W + (size_t)n0 * rb;
@@ -567,25 +576,25 @@ __global__ __launch_bounds__(QT_WAVES * WAVE) void k_qmm_tile(
 	}
 	const u32 l0 = __builtin_amdgcn_readfirstlane(lds_addr(qt_lds));
 	auto issue = [&](int s) {
-		const u32 lb = l0 + (u32)((s & 1) * G::SB + QT_XB + wave * G::J * WAVE * 4);
+		const u32 lb = l0 + (u32)((s & 1) * G::SB + G::XB + wave * G::J * WAVE * 4);
 #pragma unroll
 		for (int j = 0; j < G::J; j++)
 			dma_dword(wb + (size_t)s * G::RB, woff[j], lb + (u32)(j * WAVE * 4));
 	};
-	float4 v[4];
-	floatx16 tot[2] = {};
+	float4 v[32 / G::TPR];
+	floatx16 tot[TM] = {};
 	const int ns = K / QT_COLS;
 	auto fetch = [&](int s) {
 #pragma unroll
-		for (int j = 0; j < 4; j++)
-			v[j] = xp[(size_t)min(s, ns - 1) * (QT_COLS / 4) + 8 * j];
+		for (int j = 0; j < 32 / G::TPR; j++)
+			v[j] = xp[(size_t)min(s, ns - 1) * (QT_COLS / 4) + G::TPR * j];
 	};
 	issue(0);
 	fetch(0);
-	qt_stage(v, qt_lds, s_ts, row, i);
+	qt_stage<G::TPR, G::CHUNK>(v, qt_lds, s_ts, row, i);
 	for (int s = 0; s < ns; s++) {
 		const int b = s & 1;
-		const uint8_t *sx = qt_lds + b * G::SB, *sw = sx + QT_XB + (wn * 32 + r) * G::RB;
+		const uint8_t *sx = qt_lds + b * G::SB, *sw = sx + G::XB + (wn * 32 + r) * G::RB;
 		uint8_t *nx = qt_lds + (b ^ 1) * G::SB;
 		wait_vm<0>();    /* this wave's part of the stage's weights */
 		__syncthreads(); /* stage s is whole; the other buffer is free */
@@ -593,31 +602,31 @@ __global__ __launch_bounds__(QT_WAVES * WAVE) void k_qmm_tile(
 			issue(s + 1);
 		fetch(s + 1);
 		/* group wk: blocks GB wk .. of the stage */
-		qt_blocks<WT, GB>(sw + wk * GB * G::BB, sx + wk * 4 * GB * QT_CHUNK, s_ts + b * QT_TOK, r,
+		qt_blocks<WT, GB, TM>(sw + wk * GB * G::BB, sx + wk * 4 * GB * G::CHUNK, s_ts + b * G::TOK, r,
 				  h, tot);
 		if (s + 1 < ns)
-			qt_stage(v, nx, s_ts + (b ^ 1) * QT_TOK, row, i);
+			qt_stage<G::TPR, G::CHUNK>(v, nx, s_ts + (b ^ 1) * G::TOK, row, i);
 	}
 	if constexpr (KG > 1) { /* group 1's sums to group 0 */
 		__syncthreads();
-		float *p = (float *)qt_lds + (size_t)wn * 32 * WAVE + lane;
+		float *p = (float *)qt_lds + (size_t)wn * 16 * TM * WAVE + lane;
 		if (wk == 1) {
 #pragma unroll
-			for (int j = 0; j < 32; j++)
+			for (int j = 0; j < 16 * TM; j++)
 				p[j * WAVE] = tot[j / 16][j % 16];
 		}
 		__syncthreads();
 		if (wk == 1)
 			return;
 #pragma unroll
-		for (int j = 0; j < 32; j++)
+		for (int j = 0; j < 16 * TM; j++)
 			tot[j / 16][j % 16] += p[j * WAVE];
 	}
 	const int n = n0 + wn * 32 + r;
 	if (n >= N)
 		return;
 #pragma unroll
-	for (int t = 0; t < 2; t++)
+	for (int t = 0; t < TM; t++)
 #pragma unroll
 		for (int j = 0; j < 16; j++) {
 			const int tk = t0 + 32 * t + 8 * (j / 4) + 4 * h + j % 4;
@@ -707,43 +716,50 @@ extern "C" int moe_launch_qmm_parts(int wtype, const uint8_t *W, int N, int K, c
 	return launch_qmm(wtype, W, N, K, x, T, NULL, 0, NULL, work, true, stream);
 }
 
-template <int WT, int NW>
-static hipError_t launch_tile(const uint8_t *W, size_t rb, int N, int K, const float *x, int T,
-			      const float *add, int add_rows, float *out, hipStream_t s)
+/* 256-workgroup rounds (one per CU) of tiles of tok tokens x nr rows */
+static long long tile_rounds(int N, int T, int tok, int nr)
 {
-	typedef qt_geo<WT, NW> G;
-	const long long items = (long long)((T + QT_TOK - 1) / QT_TOK) * ((N + G::NR - 1) / G::NR);
-	if (items > 0x7fffff00ll)
-		return hipErrorInvalidValue;
-	hipLaunchKernelGGL((k_qmm_tile<WT, NW>), dim3((unsigned)((items + 7) / 8 * 8)),
-			   dim3(QT_WAVES * WAVE), 0, s, W, rb, N, K, x, T, add, add_rows, out);
-	return hipGetLastError();
+	return ((long long)((T + tok - 1) / tok) * ((N + nr - 1) / nr) + 255) / 256;
 }
 
-/* rounds of one workgroup per CU that tiles of 64 tokens x nr rows take */
-static long long tile_rounds(int N, int T, int nr)
-{
-	return ((long long)((T + QT_TOK - 1) / QT_TOK) * ((N + nr - 1) / nr) + 255) / 256;
-}
+#define SMALL_ROUNDS(N, T) tile_rounds(N, T, 32, 128)
+#define WIDE_ROUNDS(N, T) tile_rounds(N, T, 64, 256)
 
-/* 256-row tiles take 1.5 times as long as 128-row ones: 6144 x 4096 Q4_0, T =
- * 128 (48 / 96 workgroups) 89 / 63 us, T = 333 (144 / 288) 91 / 125, T = 1024
- * (384 / 768) 184 / 191 */
+/* A round of 64 x 256 tiles (one workgroup per CU) takes 95 us at K = 4096, of
+ * 32 x 128 tiles (two fit, each then half as fast) 35.  Small / wide in us,
+ * Q4_0: 6144 x 4096 T = 160 49 / 93, T = 256 71 / 96, T = 333 100 / 95, T = 1024
+ * 214 / 197; 4096 x 4096 T = 512 73 / 92, T = 1024 140 / 103; 2048 x 2048 T = 1024
+ * 41 / 54; 50304 x 2048 T = 32 40 / 52, T = 48 72 / 55.  (64 x 128 tiles, one per
+ * CU, were never more than a tenth better than both.) */
 static bool tile_wide(int N, int T)
 {
-	return 3 * tile_rounds(N, T, 256) <= 2 * tile_rounds(N, T, 128);
+	return 8 * WIDE_ROUNDS(N, T) < 3 * SMALL_ROUNDS(N, T);
 }
 
 /* Whether moe_launch_qmm_tile is faster than moe_launch_qmm: a workgroup of
  * k_qmm (16 tokens, 64 rows, 512 columns) takes about 22 ns of the whole
- * chip, a round of tiles 13.1 (128 rows) or 20.5 ns (256 rows) per column of
- * K.  k_qmm / tiles in us: 6144 x 4096 T = 48 54 / 55, T = 64 67 / 56; 4096 x
- * 4096 T = 64 49 / 54; 2048 x 2048 T = 64 17 / 30, T = 512 78 / 33; 50304 x 2048
- * T = 16 71 / 56; 32000 x 4096 T = 2 76 / 75, T = 16 86 / 77 */
+ * chip, a round of tiles 9.8 (small) or 23 ns (wide) per column of K.  k_qmm /
+ * tiles in us: 6144 x 4096 T = 17 36 / 38, T = 33 51 / 39; 4096 x 4096 T = 48
+ * 39 / 39, T = 64 49 / 39; 2048 x 2048 T = 64 17 / 22; 6144 x 2048 T = 32 22 / 22,
+ * T = 48 32 / 22; 50304 x 2048 T = 2 62 / 35, T = 16 71 / 39; 32000 x 4096 T = 2
+ * 76 / 45, T = 16 86 / 48 */
 extern "C" int moe_qmm_tile_better(int N, int T)
 {
 	const long long w = (long long)((T + QMM_TOK - 1) / QMM_TOK) * ((N + 63) / 64);
-	return w > 305 * tile_rounds(N, T, 128) || w > 477 * tile_rounds(N, T, 256);
+	return w > 228 * SMALL_ROUNDS(N, T) || w > 540 * WIDE_ROUNDS(N, T);
+}
+
+template <int WT, int NW, int TM>
+static hipError_t launch_tile(const uint8_t *W, size_t rb, int N, int K, const float *x, int T,
+			      const float *add, int add_rows, float *out, hipStream_t s)
+{
+	typedef qt_geo<WT, NW, TM> G;
+	const long long items = (long long)((T + G::TOK - 1) / G::TOK) * ((N + G::NR - 1) / G::NR);
+	if (items > 0x7fffff00ll)
+		return hipErrorInvalidValue;
+	hipLaunchKernelGGL((k_qmm_tile<WT, NW, TM>), dim3((unsigned)((items + 7) / 8 * 8)),
+			   dim3(QT_WAVES * WAVE), 0, s, W, rb, N, K, x, T, add, add_rows, out);
+	return hipGetLastError();
 }
 
 extern "C" int moe_launch_qmm_tile(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
@@ -753,10 +769,9 @@ extern "C" int moe_launch_qmm_tile(int wtype, const uint8_t *W, int N, int K, co
 		return (int)hipErrorInvalidValue;
 	const size_t rb = (size_t)(K / 32) * (wtype == 1 ? 34 : 18);
 	hipStream_t s = (hipStream_t)stream;
-	const long long tiles = (T + QT_TOK - 1) / QT_TOK;
 	if (tile_wide(N, T))
-		return (int)(wtype == 1 ? launch_tile<1, 8>(W, rb, N, K, x, T, add, add_rows, out, s)
-					: launch_tile<2, 8>(W, rb, N, K, x, T, add, add_rows, out, s));
-	return (int)(wtype == 1 ? launch_tile<1, 4>(W, rb, N, K, x, T, add, add_rows, out, s)
-				: launch_tile<2, 4>(W, rb, N, K, x, T, add, add_rows, out, s));
+		return (int)(wtype == 1 ? launch_tile<1, 8, 2>(W, rb, N, K, x, T, add, add_rows, out, s)
+					: launch_tile<2, 8, 2>(W, rb, N, K, x, T, add, add_rows, out, s));
+	return (int)(wtype == 1 ? launch_tile<1, 4, 1>(W, rb, N, K, x, T, add, add_rows, out, s)
+				: launch_tile<2, 4, 1>(W, rb, N, K, x, T, add, add_rows, out, s));
 }

@@ -1,5 +1,5 @@
-"""The Q8_0/Q4_0 product of many tokens in tiles (64 tokens, 128 or 256 rows,
-stages of 128 columns) at the edges of its tiles, against float64."""
+"""The Q8_0/Q4_0 product of many tokens in tiles (32 tokens x 128 rows or 64 x
+256, stages of 128 columns) at the edges of its tiles, against float64."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # remainders; the fewest columns; many rows at two tokens; a chip-filling grid
 @pytest.mark.parametrize("wt", (hipmoe.Q8_0, hipmoe.Q4_0))
 @pytest.mark.parametrize("N,K,Ts", ((1, 256, (65,)), (129, 512, (128, 129)), (257, 4096, (191,)),
-                                    (20000, 256, (2, 17, 130)), (2100, 1024, (1025,))))
+                                    (20000, 256, (2, 33, 130)), (2100, 1024, (1025,))))
 def test_gpu_qmm_tile_vs_float64(wt, N, K, Ts):
     q = hipmoe.synth_quant_matrix(SEED, 41, 0.02, wt, N, K)
     w = oracle.dequant(np.frombuffer(q, np.uint8), wt, N * K).reshape(N, K).astype(np.float64)
