@@ -414,7 +414,8 @@ hip_lm *hip_lm_upload(const hip_lm_desc *d)
 
 	HIPCHK(hipGetDevice(&M->device), "hipGetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&M->stream, hipStreamNonBlocking), "hipStreamCreate");
-	HIPCHK(hipHostMalloc((void **)&M->h_io, (16 + M->V) * sizeof(float), 0), "hipHostMalloc");
+	HIPCHK(hipHostMalloc((void **)&M->h_io, (16 + M->V) * sizeof(float),
+			     hipHostMallocPortable), "hipHostMalloc");
 	HIPCHK(hipEventCreate(&M->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&M->ev1), "hipEventCreate");
 
@@ -1382,9 +1383,11 @@ hip_lm_batch *hip_lm_batch_new(hip_lm *M, size_t nseq)
 	const size_t part = S * M->H * (size_t)M->nch * (LM_HLEN + 2) * sizeof(uint64_t);
 	HIPCHK(hipSetDevice(M->device), "hipSetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking), "hipStreamCreate");
-	HIPCHK(hipHostMalloc((void **)&B->h_io, (LM_REPORT_WORDS + S) * sizeof(int), 0), "hipHostMalloc");
+	HIPCHK(hipHostMalloc((void **)&B->h_io, (LM_REPORT_WORDS + S) * sizeof(int),
+			     hipHostMallocPortable), "hipHostMalloc");
 	if (S * M->V * sizeof(float) <= BATCH_PINNED)
-		HIPCHK(hipHostMalloc((void **)&B->h_logits, S * M->V * sizeof(float), 0),
+		HIPCHK(hipHostMalloc((void **)&B->h_logits, S * M->V * sizeof(float),
+				     hipHostMallocPortable),
 		       "hipHostMalloc");
 	HIPCHK(hipEventCreate(&B->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&B->ev1), "hipEventCreate");

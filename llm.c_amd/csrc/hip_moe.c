@@ -1008,7 +1008,8 @@ static int ffn_pinned(hip_moe_layer *L, const float *x, float *out, size_t T,
 	/* per token: x, out, ids, weights; the bias and the error word */
 	const size_t in = most * L->E + L->NE, res = most * (L->E + 2 * L->topk) + 1;
 	if (!L->h_io) {
-		if (hipHostMalloc((void **)&L->h_io, (in + res) * sizeof(float), 0) != hipSuccess) {
+		if (hipHostMalloc((void **)&L->h_io, (in + res) * sizeof(float),
+				  hipHostMallocPortable) != hipSuccess) {
 			L->h_io = NULL;
 			return -1;
 		}
