@@ -283,8 +283,8 @@ hip_moe_qmat *hip_moe_qmat_upload(const void *qdata, int wtype, size_t N, size_t
  * absolute error per output within 2^-24 * (32 (127 + c) + 31 c + 64 * 255)
  * * (sum over blocks of |d| * sum |x|) to first order; ~1e-6 relative L2 on
  * zero-mean activations.  Several tokens (T >= 2) of a Q8_0/Q4_0 matrix run
- * on the matrix cores instead: each token's 32 (few tokens) or 128 values
- * scaled by a power of two and split into two f16 parts (~22 bits together), the quants
+ * on the matrix cores instead: each 32-value token block scaled by a power
+ * of two and split into two f16 parts (~22 bits together), the quants
  * unscaled (exact in f16), the block scale applied per block in fp32, so the
  * outputs keep fp32 accuracy (~1e-7 relative, summation order only).
  * Q4_K/Q6_K matrices take the reference's Q8_K

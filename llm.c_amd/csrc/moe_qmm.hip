@@ -42,8 +42,8 @@
  * launches at 16 tokens x 6144 x 4096 Q4_0: the last arrivals' polls sit
  * in series behind the slowest stretch.)
  *
- * Many tokens, or very many rows, take k_qmm_tile below: tiles of 32 or 64 tokens
- * over the whole of K, the tokens scaled per 128 columns.
+ * Many tokens, or very many rows, take k_qmm_tile below: tiles of 32 or 64
+ * tokens over the whole of K, the same split with a scale per block.
  *
  * Bound of k_qmm: HBM for a few tokens (the weights are read once per token tile;
  * the tokens, T * K * 4 bytes, come from L2).  Algorithmic bytes per call:
@@ -311,7 +311,7 @@ template <int WT, int NW, int TM> struct qt_geo {
 	static constexpr int J = (NR * DW + QT_WAVES * WAVE - 1) / (QT_WAVES * WAVE);
 	static constexpr int WB = J * QT_WAVES * WAVE * 4;
 	static constexpr int SB = XB + WB; /* one stage */
-	static constexpr int LDS = 2 * SB + 2 * TOK * 4;
+	static constexpr int LDS = 2 * SB + 2 * 4 * TOK * 4; /* and the scales of its blocks */
 };
 
 /* a lane's share of block b (parity ODD) of its row's stage in LDS: raw
@@ -392,31 +392,50 @@ template <int ODD> struct qt_blk<1, ODD> {
 
 /*
  * NBK blocks of a stage for one wave: 32 TM tokens x 32 rows, each block's sums
- * scaled by the row's block scale, their total by the tokens' scales into
- * tot.  Software-pipelined by hand in steps of half a block (its hi, then its
- * lo operands): a step's MFMAs run beside the next step's LDS reads, the
- * fp32 steps of the block before and the unpacking of the block after (left
- * to itself the compiler reads each operand right before its MFMA and waits
- * out the LDS latency every time).
+ * scaled by the row's block scale and the tokens' (their product is exact)
+ * and added to acc.  In steps of half a block, ordered by hand: a step's MFMAs
+ * run beside the next step's LDS reads and the unpacking of the block after
+ * (left to itself the compiler reads each operand right before its MFMA and
+ * waits out the LDS latency every time).  TM = 2: a step is a group of 32
+ * tokens, and the fp32 steps of the last one's sums stand beside its MFMAs.
+ * TM = 1: a step is the hi or the lo operands, and the last block's fp32 steps
+ * come before the next one's MFMAs (the SIMD's other waves fill in; a second
+ * set of sums, beside the 128 registers of two workgroups a CU, spilled).
  */
 template <int WT, int NBK, int TM>
 __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, const float *sts, int r,
-					int h, floatx16 (&tot)[TM])
+					int h, floatx16 (&acc)[TM])
 {
-	constexpr int BB = qt_geo<WT, 8, TM>::BB, CH = qt_geo<WT, 8, TM>::CHUNK;
+	constexpr int BB = qt_geo<WT, 8, TM>::BB, CH = qt_geo<WT, 8, TM>::CHUNK, TOK = 32 * TM;
+	constexpr int NQ = 2 * TM; /* MFMAs of a step */
 	qt_blk<WT, 0> we;
 	qt_blk<WT, 1> wo;
-	half8_t k[2][2], a[2][2][TM]; /* k: [block & 1][kh]; a: [step & 1][kh][t] */
-	floatx16 s[2][TM], acc[TM];
+	half8_t k[2][2], a[2][NQ]; /* k: [block & 1][kh]; a: [step & 1][kh, and hi or lo] */
+	floatx16 s[TM];
+	floatx4 ts[TM][4]; /* scales of the lane's tokens 8 i + 4 h .. + 3 of a group */
 	float d[2];
 	auto reada = [&](int step) {
-		const int b = step / 2, p = step % 2;
+		const int b = step / 2, u = step % 2;
 #pragma unroll
-		for (int kh = 0; kh < 2; kh++)
+		for (int q = 0; q < NQ; q++) {
+			const int p = TM == 2 ? q / 2 : u, kh = q % 2, t = TM == 2 ? u : 0;
+			a[step & 1][q] = *(const half8_t *)(sx + (16 * p + 4 * b + 2 * kh + h) * CH +
+							    (32 * t + r) * 16);
+		}
+	};
+	auto readts = [&](int b, int t) {
 #pragma unroll
-			for (int t = 0; t < TM; t++)
-				a[step & 1][kh][t] = *(const half8_t *)(
-					sx + (16 * p + 4 * b + 2 * kh + h) * CH + (32 * t + r) * 16);
+		for (int i = 0; i < 4; i++)
+			ts[t][i] = *(const floatx4 *)(sts + b * TOK + 32 * t + 8 * i + 4 * h);
+	};
+	/* acc += the sums of block b and token group t, scaled */
+	auto add = [&](int b, int t) {
+#pragma unroll
+		for (int j = 0; j < 16; j++)
+			acc[t][j] = __builtin_fmaf(d[b & 1] * ts[t][j / 4][j % 4], s[t][j], acc[t][j]);
+		/* in this step: left to itself the compiler puts every block's fp32
+		 * steps behind the last MFMA and spills the sums until then */
+		asm volatile("" : "+v"(acc[t]));
 	};
 	we.load(row, h);
 	wo.load(row + BB, h);
@@ -425,10 +444,14 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 	__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
 	for (int step = 0; step < 2 * NBK; step++) {
-		const int b = step / 2, p = step % 2, f = b & 1;
+		const int b = step / 2, u = step % 2, f = b & 1, t = TM == 2 ? u : 0;
 		if (step + 1 < 2 * NBK)
 			reada(step + 1);
-		if (p == 0) { /* block b + 2's bytes, over block b's, which k holds */
+		if (TM == 2)
+			readts(b, u);
+		else if (u == 0 && b > 0)
+			readts(b - 1, 0);
+		if (u == 0) { /* block b + 2's bytes, over block b's, which k holds */
 			if (b + 2 < NBK) {
 				if (f == 0)
 					we.load(row + (b + 2) * BB, h);
@@ -441,90 +464,69 @@ __device__ static inline void qt_blocks(const uint8_t *row, const uint8_t *sx, c
 			else
 				we.operands(k[0], d[0]);
 		}
+		if (TM == 1 && u == 0 && b > 0)
+			add(b - 1, 0);
 #pragma unroll
-		for (int kh = 0; kh < 2; kh++)
-#pragma unroll
-			for (int t = 0; t < TM; t++) {
-				const floatx16 z = {};
-				s[f][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-					a[step & 1][kh][t], k[f][kh], p == 0 && kh == 0 ? z : s[f][t], 0, 0, 0);
-			}
-		if (b > 0 && p == 0) { /* the block before (the next step's unpacking replaces d) */
-			const float e = d[f ^ 1];
-#pragma unroll
-			for (int t = 0; t < TM; t++)
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-					acc[t][j] = b == 1 ? e * s[f ^ 1][t][j]
-							   : __builtin_fmaf(e, s[f ^ 1][t][j], acc[t][j]);
+		for (int q = 0; q < NQ; q++) {
+			const floatx16 z = {};
+			s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+				a[step & 1][q], k[f][q % 2], q == 0 && (TM == 2 || u == 0) ? z : s[t], 0, 0, 0);
 		}
+		if (TM == 2 && step > 0) /* the next step's unpacking replaces its d */
+			add((step - 1) / 2, (step - 1) % 2);
 		__builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
 #pragma unroll
-		for (int i = 0; i < 2 * TM; i++) {
+		for (int i = 0; i < NQ; i++) {
 			__builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-			__builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+			__builtin_amdgcn_sched_group_barrier(0x2, 16, 0);
 		}
 		__builtin_amdgcn_sched_barrier(0);
 	}
-	const floatx4 *ts = (const floatx4 *)(sts + 4 * h);
-	constexpr int f = (NBK - 1) & 1;
-#pragma unroll
-	for (int t = 0; t < TM; t++)
-#pragma unroll
-		for (int j = 0; j < 16; j++)
-			tot[t][j] = __builtin_fmaf(ts[8 * t + 2 * (j / 4)][j % 4],
-						   __builtin_fmaf(d[f], s[f][t][j], acc[t][j]), tot[t][j]);
+	if (TM == 1)
+		readts(NBK - 1, 0);
+	add(NBK - 1, TM - 1);
+}
+
+/* the maximum over eight neighbouring lanes: lanes ^ 1, ^ 2, the other four
+ * mirrored */
+__device__ static inline u32 qt_max8(u32 m)
+{
+	m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0xb1, 0xf, 0xf, true));
+	m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x4e, 0xf, 0xf, true));
+	return max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xf, 0xf, true));
 }
 
 /*
  * A token's 128 columns of a stage, held by TPR = 8 or 16 threads (thread i:
- * the float4s i, i + TPR, ...), scaled by one power of two (the largest
- * magnitude into [2^13, 2^14)) and split into hi and lo.
+ * the float4s i, i + TPR, ...: eight neighbouring threads hold a block), each
+ * block scaled by a power of two of its own (its largest magnitude into
+ * [2^13, 2^14)) and split into hi and lo.  Scales stop at 2^125: below that
+ * all bits of a value fit the two parts, and the inverse times a weight's f16
+ * scale is exact in fp32.
  */
-template <int TPR, int CH>
+template <int TPR, int CH, int TOK>
 __device__ static inline void qt_stage(const float4 (&v)[32 / TPR], uint8_t *sx, float *ts, int row, int i)
 {
 	typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-	float m = 0.0f;
 #pragma unroll
 	for (int j = 0; j < 32 / TPR; j++) {
-		m = fmaxf(fmaxf(m, fabsf(v[j].x)), fabsf(v[j].y));
-		m = fmaxf(fmaxf(m, fabsf(v[j].z)), fabsf(v[j].w));
-	}
-	/* the threads' maximum: lanes ^ 1, ^ 2, the other four mirrored, the other
-	 * eight mirrored */
-	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0xb1,
-									0xf, 0xf, true)));
-	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x4e,
-									0xf, 0xf, true)));
-	m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, m), 0x141,
-									0xf, 0xf, true)));
-	if constexpr (TPR == 16)
-		m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(
-						   __builtin_bit_cast(int, m), 0x140, 0xf, 0xf, true)));
-	int sh = 0;
-	if (m > 0.0f) { /* 13 - exponent; the largest scale a float holds below that */
-		sh = 140 - (int)((__builtin_bit_cast(u32, m) >> 23) & 0xffu);
-		sh = sh > 126 ? 126 : sh;
-	}
-	const float s = __builtin_bit_cast(float, (u32)(sh + 127) << 23);
-#pragma unroll
-	for (int j = 0; j < 32 / TPR; j++) {
+		/* magnitudes compare as their bits do */
+		const u32 m = qt_max8(__builtin_bit_cast(
+			u32, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w)))));
+		/* exponent 13 - m's, 125 at most (a zero block's too) */
+		const u32 sb = min((267u << 23) - (m & 0x7f800000u), 252u << 23);
+		const float s = __builtin_bit_cast(float, sb);
 		/* element order 0, 2, 1, 3: a weight operand's */
-		const float y[4] = {v[j].x * s, v[j].z * s, v[j].y * s, v[j].w * s};
-		half4_t hi, lo;
-#pragma unroll
-		for (int k = 0; k < 4; k++) {
-			hi[k] = (_Float16)y[k];
-			lo[k] = (_Float16)(y[k] - (float)hi[k]);
-		}
+		const floatx4 y = {v[j].x * s, v[j].z * s, v[j].y * s, v[j].w * s};
+		const half4_t hi = __builtin_convertvector(y, half4_t);
+		const half4_t lo = __builtin_convertvector(y - __builtin_convertvector(hi, floatx4), half4_t);
 		const int f = i + TPR * j; /* of the token's 32 float4s: block f / 8 */
 		uint8_t *o = sx + (f >> 1) * CH + row * 16 + (f & 1) * 8;
 		*(half4_t *)o = hi;
 		*(half4_t *)(o + 16 * CH) = lo;
+		if (f % 8 == 0)
+			ts[(f / 8) * TOK + row] = __builtin_bit_cast(float, (254u << 23) - sb);
 	}
-	if (i == 0)
-		ts[row] = __builtin_bit_cast(float, (u32)(127 - sh) << 23);
 }
 
 /*
@@ -536,14 +538,21 @@ __device__ static inline void qt_stage(const float4 (&v)[32 / TPR], uint8_t *sx,
  * of two buffers: one barrier a stage, and no scratch memory, so calls on one
  * matrix may overlap and be captured.
  *
- * Bound: the VALU (the tokens' split, the unpacking, one fp32 step per block
- * and output) and the MFMAs, each about 2,500 cycles of a 64 x 256 stage's
- * 6,000, in a single workgroup per CU (LDS); two 32 x 128 ones fit.  Q4_0 6144 x 4096, 333 tokens: 926 -> 85 us
- * (the per-token product, which takes the weights once per token), 1024
- * tokens against k_qmm 908 -> 184; 4096 x 4096, 1024 tokens 608 -> 101.  Tried:
- * 32 tokens x 64 rows a wave (half the operand reads, twice the unpacking)
- * 91 -> 101; splitting the tokens at opposite ends of a stage in a SIMD's two
- * waves 91 -> 96; without the hand-pipelined order 104.
+ * Bound: the VALU (the tokens' split, the unpacking, a multiplication and an
+ * FMA per block and output) and the MFMAs, which overlap only in part: about
+ * 500 and 32 instructions a wave of a 64 x 256 stage, 4,000 and 2,050 of its
+ * 7,000 cycles, in a single workgroup per CU (LDS); two 32 x 128 ones fit.
+ * Q4_0 6144 x 4096, calls back to back: 333 tokens 926 -> 94 us (the per-token
+ * product, which takes the weights once per token), 1024 tokens against
+ * k_qmm 908 -> 190; 4096 x 4096, 1024 tokens 608 -> 106.  One scale per token
+ * and 128 columns would save the multiplications (333 tokens 88, 1024 tokens
+ * 171) but cost the blocks below their neighbours bits.  Tried with that form
+ * at 333 tokens (91 there): 32 tokens x 64 rows a wave (half the operand reads,
+ * twice the unpacking) 101; splitting the tokens at opposite ends of a stage
+ * in a SIMD's two waves 96; without the hand-made order 104.  Tried with this
+ * one: the scales as a byte each in LDS (a quarter of their reads, a shift
+ * more per output) 128; the tokens' loads where the compiler puts them, right
+ * before their use, 103.
  */
 template <int WT, int NW, int TM>
 __global__ __launch_bounds__(QT_WAVES * WAVE, TM == 1 ? 4 : 2) void k_qmm_tile(
@@ -553,7 +562,7 @@ __global__ __launch_bounds__(QT_WAVES * WAVE, TM == 1 ? 4 : 2) void k_qmm_tile(
 	typedef qt_geo<WT, NW, TM> G;
 	constexpr int KG = QT_WAVES / NW, GB = 4 / KG; /* K groups; blocks of a stage each takes */
 	__shared__ __attribute__((aligned(16))) uint8_t qt_lds[G::LDS];
-	float *s_ts = (float *)(qt_lds + 2 * G::SB); /* [2][64] */
+	float *s_ts = (float *)(qt_lds + 2 * G::SB); /* [2][4][TOK] */
 	const int tid = threadIdx.x, lane = tid % WAVE;
 	const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
 	const int r = lane & 31, h = lane >> 5, wn = wave % NW, wk = wave / NW;
@@ -591,21 +600,32 @@ __global__ __launch_bounds__(QT_WAVES * WAVE, TM == 1 ? 4 : 2) void k_qmm_tile(
 	};
 	issue(0);
 	fetch(0);
-	qt_stage<G::TPR, G::CHUNK>(v, qt_lds, s_ts, row, i);
-	for (int s = 0; s < ns; s++) {
-		const int b = s & 1;
-		const uint8_t *sx = qt_lds + b * G::SB, *sw = sx + G::XB + (wn * 32 + r) * G::RB;
-		uint8_t *nx = qt_lds + (b ^ 1) * G::SB;
-		wait_vm<0>();    /* this wave's part of the stage's weights */
-		__syncthreads(); /* stage s is whole; the other buffer is free */
-		if (s + 1 < ns)
-			issue(s + 1);
-		fetch(s + 1);
-		/* group wk: blocks GB wk .. of the stage */
-		qt_blocks<WT, GB, TM>(sw + wk * GB * G::BB, sx + wk * 4 * GB * G::CHUNK, s_ts + b * G::TOK, r,
-				  h, tot);
-		if (s + 1 < ns)
-			qt_stage<G::TPR, G::CHUNK>(v, nx, s_ts + (b ^ 1) * G::TOK, row, i);
+	qt_stage<G::TPR, G::CHUNK, G::TOK>(v, qt_lds, s_ts, row, i);
+	for (int s = 0; s < ns;) {
+		/* sums of 512 columns first, as k_qmm's: a chain over all of K = 4096
+		 * left 1.32e-7 (relative L2 against float64), these 1.06e-7, k_qmm 1.15e-7 */
+		floatx16 acc[TM] = {};
+#pragma unroll 1
+		for (const int e = min(s + 4, ns); s < e; s++) {
+			const int b = s & 1;
+			const uint8_t *sx = qt_lds + b * G::SB, *sw = sx + G::XB + (wn * 32 + r) * G::RB;
+			uint8_t *nx = qt_lds + (b ^ 1) * G::SB;
+			wait_vm<0>();    /* this wave's part of the stage's weights */
+			__syncthreads(); /* stage s is whole; the other buffer is free */
+			if (s + 1 < ns)
+				issue(s + 1);
+			fetch(s + 1);
+			__builtin_amdgcn_sched_barrier(0); /* not down to their use */
+			/* group wk: blocks GB wk .. of the stage */
+			qt_blocks<WT, GB, TM>(sw + wk * GB * G::BB, sx + wk * 4 * GB * G::CHUNK,
+					      s_ts + (4 * b + wk * GB) * G::TOK, r, h, acc);
+			/* the last stage's is not read: under a condition the compiler would
+			 * move the loads there, and the wait for them */
+			qt_stage<G::TPR, G::CHUNK, G::TOK>(v, nx, s_ts + 4 * (b ^ 1) * G::TOK, row, i);
+		}
+#pragma unroll
+		for (int t = 0; t < TM; t++)
+			tot[t] += acc[t];
 	}
 	if constexpr (KG > 1) { /* group 1's sums to group 0 */
 		__syncthreads();
@@ -725,12 +745,13 @@ static long long tile_rounds(int N, int T, int tok, int nr)
 #define SMALL_ROUNDS(N, T) tile_rounds(N, T, 32, 128)
 #define WIDE_ROUNDS(N, T) tile_rounds(N, T, 64, 256)
 
-/* A round of 64 x 256 tiles (one workgroup per CU) takes 95 us at K = 4096, of
- * 32 x 128 tiles (two fit, each then half as fast) 35.  Small / wide in us,
- * Q4_0: 6144 x 4096 T = 160 49 / 93, T = 256 71 / 96, T = 333 100 / 95, T = 1024
- * 214 / 197; 4096 x 4096 T = 512 73 / 92, T = 1024 140 / 103; 2048 x 2048 T = 1024
- * 41 / 54; 50304 x 2048 T = 32 40 / 52, T = 48 72 / 55.  (64 x 128 tiles, one per
- * CU, were never more than a tenth better than both.) */
+/* A round of 64 x 256 tiles (one workgroup per CU) takes 93 us at K = 4096, of
+ * 32 x 128 tiles (two fit, each then half as fast) 35.  Small / wide in us
+ * (calls back to back), Q4_0: 6144 x 4096 T = 160 47 / 93, T = 256 69 / 94, T =
+ * 333 98 / 93, T = 768 168 / 189, T = 1024 213 / 192; 4096 x 4096 T = 512 72 / 94,
+ * T = 768 112 / 101, T = 1024 144 / 106; 2048 x 2048 T = 1024 38 / 52; 50304 x 2048
+ * T = 32 36 / 52, T = 48 67 / 52; 32000 x 4096 T = 48 70 / 94.  (64 x 128 tiles, one
+ * per CU, were never more than a tenth better than both.) */
 static bool tile_wide(int N, int T)
 {
 	return 8 * WIDE_ROUNDS(N, T) < 3 * SMALL_ROUNDS(N, T);
@@ -739,10 +760,10 @@ static bool tile_wide(int N, int T)
 /* Whether moe_launch_qmm_tile is faster than moe_launch_qmm: a workgroup of
  * k_qmm (16 tokens, 64 rows, 512 columns) takes about 22 ns of the whole
  * chip, a round of tiles 9.8 (small) or 23 ns (wide) per column of K.  k_qmm /
- * tiles in us: 6144 x 4096 T = 17 36 / 38, T = 33 51 / 39; 4096 x 4096 T = 48
- * 39 / 39, T = 64 49 / 39; 2048 x 2048 T = 64 17 / 22; 6144 x 2048 T = 32 22 / 22,
- * T = 48 32 / 22; 50304 x 2048 T = 2 62 / 35, T = 16 71 / 39; 32000 x 4096 T = 2
- * 76 / 45, T = 16 86 / 48 */
+ * tiles in us, Q4_0, calls back to back: 6144 x 4096 T = 17 36 / 39, T = 33 50 /
+ * 40; 4096 x 4096 T = 48 38 / 40, T = 64 48 / 40; 2048 x 2048 T = 64 17 / 22; 6144 x
+ * 2048 T = 32 22 / 22, T = 33 30 / 22; 50304 x 2048 T = 2 60 / 36, T = 16 69 / 37;
+ * 32000 x 4096 T = 2 73 / 42, T = 16 83 / 43 */
 extern "C" int moe_qmm_tile_better(int N, int T)
 {
 	const long long w = (long long)((T + QMM_TOK - 1) / QMM_TOK) * ((N + 63) / 64);
