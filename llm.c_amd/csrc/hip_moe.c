@@ -63,7 +63,7 @@ struct hip_moe_layer {
 	void *d_h16;        /* grouped path: f16 h in sorted row order */
 	void *d_xh;         /* grouped path: tokens rounded to f16 [T][E] */
 	void *d_rec;        /* K-quant experts, many tokens: their Q8_K records */
-	float *d_hs;        /* and h in sorted row order */
+	size_t kq_T;        /* tokens of the grouped K-quant products' scratch */
 
 	/* staging for the host-pointer entry point */
 	size_t cap_io;
@@ -224,7 +224,6 @@ void hip_moe_free(hip_moe_layer *L)
 	hipFree(L->d_h16);
 	hipFree(L->d_xh);
 	hipFree(L->d_rec);
-	hipFree(L->d_hs);
 	hipFree(L->d_x);
 	hipFree(L->d_out);
 	hipFree(L->d_bias);
@@ -377,7 +376,7 @@ size_t hip_moe_weight_bytes(const hip_moe_layer *L)
 }
 
 /* 32-row tiles a sort of P pairs can use, and whether the grouped K-quant
- * products (kq_grouped.hip) take a call of T tokens.  The other kernels read
+ * products (kq_grouped.hip) are the faster ones for T tokens.  The other kernels read
  * an expert's weights once per pair, these once per expert and 32 pairs but
  * in five more launches: taken once the pairs past one per expert would
  * re-read KQ_GROUPED_BYTES.  Measured either side of it (Q4_K gate/up, Q6_K
@@ -392,13 +391,44 @@ static size_t kq_tiles(const hip_moe_layer *L, size_t P)
 	return (P + r - 1) / r + (L->NE < P ? L->NE : P);
 }
 
-static int kq_grouped_fits(const hip_moe_layer *L, size_t T)
+static int kq_grouped_worth(const hip_moe_layer *L, size_t T)
 {
 	const size_t P = T * L->topk;
 	return P > L->NE &&
-	       (P - L->NE) * (2 * L->gu_stride + L->down_stride) >= KQ_GROUPED_BYTES &&
-	       kq_tiles(L, P) <= (size_t)moe_prefill_tile_cap() &&
-	       moe_kq_rec_bytes(T, L->E) <= 0xffffffffull;
+	       (P - L->NE) * (2 * L->gu_stride + L->down_stride) >= KQ_GROUPED_BYTES;
+}
+
+/* the most tokens those products take: the sort's tile table, 32-bit offsets
+ * into the records */
+static size_t kq_grouped_most(const hip_moe_layer *L)
+{
+	const size_t tiles = (size_t)moe_prefill_tile_cap() - L->NE;
+	const size_t a = tiles * (size_t)moe_kq_tile_rows() / L->topk;
+	const size_t b = 0xffffffffull / moe_kq_rec_bytes(1, L->E);
+	return a < b ? a : b;
+}
+
+/* their buffers for T tokens, with one h for the P pairs of the other
+ * kernels and their padded rows; without the memory none (a call then takes
+ * the other kernels) */
+static int kq_grouped_alloc(hip_moe_layer *L, size_t T, size_t P)
+{
+	const size_t tiles = kq_tiles(L, T * L->topk), rows = tiles * (size_t)moe_kq_tile_rows();
+	if (hipMalloc((void **)&L->d_h, (P > rows ? P : rows) * L->EI * sizeof(float)) == hipSuccess &&
+	    hipMalloc((void **)&L->d_rows, rows * sizeof(int)) == hipSuccess &&
+	    hipMalloc((void **)&L->d_tile_e, (tiles + 1) * sizeof(int)) == hipSuccess &&
+	    hipMalloc(&L->d_rec, moe_kq_rec_bytes(T, L->E)) == hipSuccess)
+		return 1;
+	(void)hipGetLastError(); /* the launches check it */
+	hipFree(L->d_h);
+	hipFree(L->d_rows);
+	hipFree(L->d_tile_e);
+	hipFree(L->d_rec);
+	L->d_h = NULL;
+	L->d_rows = NULL;
+	L->d_tile_e = NULL;
+	L->d_rec = NULL;
+	return 0;
 }
 
 /*
@@ -433,11 +463,9 @@ static int ensure_scratch(hip_moe_layer *L, size_t T, hipStream_t s)
 	hipFree(L->d_h16);
 	hipFree(L->d_xh);
 	hipFree(L->d_rec);
-	hipFree(L->d_hs);
 	L->d_part = NULL;
 	L->d_xh = NULL;
 	L->d_rec = NULL;
-	L->d_hs = NULL;
 	L->d_rows = NULL;
 	L->d_tile_e = NULL;
 	L->d_h16 = NULL;
@@ -448,10 +476,10 @@ static int ensure_scratch(hip_moe_layer *L, size_t T, hipStream_t s)
 	L->d_ypart = NULL;
 	L->d_sync = NULL;
 	L->cap_T = 0;
+	L->kq_T = 0;
 	HIPCHK(hipMalloc((void **)&L->d_logits, T * L->NE * sizeof(float)), "hipMalloc(logits)");
 	HIPCHK(hipMalloc((void **)&L->d_ids, P * sizeof(uint32_t)), "hipMalloc(ids)");
 	HIPCHK(hipMalloc((void **)&L->d_w, P * sizeof(float)), "hipMalloc(w)");
-	HIPCHK(hipMalloc((void **)&L->d_h, P * L->EI * sizeof(float)), "hipMalloc(h)");
 	/* fp32 partials of the GEMV (its K-chunks) and grouped paths (their
 	 * K-splits: room for several when the pairs are few) */
 	L->ypart_cap = moe_down_part_floats(L->E, L->EI, P);
@@ -488,17 +516,14 @@ static int ensure_scratch(hip_moe_layer *L, size_t T, hipStream_t s)
 		HIPCHK(hipMalloc(&L->d_h16, rows * L->EI * 2), "hipMalloc(h16)");
 		HIPCHK(hipMalloc(&L->d_xh, T * L->E * 2), "hipMalloc(xh)");
 	}
-	if (L->kq && kq_grouped_fits(L, T)) {
-		const size_t tiles = kq_tiles(L, P);
-		HIPCHK(hipMalloc((void **)&L->d_rows, tiles * moe_kq_tile_rows() * sizeof(int)),
-		       "hipMalloc(rows)");
-		HIPCHK(hipMalloc((void **)&L->d_tile_e, (tiles + 1) * sizeof(int)),
-		       "hipMalloc(tiles)");
-		HIPCHK(hipMalloc((void **)&L->d_hs,
-				 tiles * moe_kq_tile_rows() * L->EI * sizeof(float)),
-		       "hipMalloc(sorted h)");
-		HIPCHK(hipMalloc(&L->d_rec, moe_kq_rec_bytes(T, L->E)), "hipMalloc(records)");
+	/* after what every call needs */
+	if (L->kq) {
+		const size_t most = kq_grouped_most(L), t = T < most ? T : most;
+		if (kq_grouped_worth(L, t) && kq_grouped_alloc(L, t, P))
+			L->kq_T = t;
 	}
+	if (!L->d_h)
+		HIPCHK(hipMalloc((void **)&L->d_h, P * L->EI * sizeof(float)), "hipMalloc(h)");
 	L->cap_T = T;
 	L->scratch_gen++;
 	return 1;
@@ -849,7 +874,7 @@ int hip_moe_ffn_dev(hip_moe_layer *L, const float *d_x, float *d_out, size_t T,
 		set_err("ffn: the requested path does not apply to this layer and T=%zu", T);
 		return 0;
 	}
-	if (L->kq && L->path == HIP_MOE_PATH_AUTO && L->d_rec && kq_grouped_fits(L, T)) {
+	if (L->kq && L->path == HIP_MOE_PATH_AUTO && T <= L->kq_T && kq_grouped_worth(L, T)) {
 		const int tiles = (int)kq_tiles(L, (size_t)P);
 		if (!route(L, d_x, T, d_router_bias, L->d_logits, NULL, ids, w, NULL, s))
 			return 0;
@@ -858,7 +883,7 @@ int hip_moe_ffn_dev(hip_moe_layer *L, const float *d_x, float *d_out, size_t T,
 		     "sort by expert");
 		LCHK(moe_launch_kq_grouped(L->wtype, L->dtype, L->d_gate, L->d_up, L->d_down,
 					   L->gu_stride, L->down_stride, L->d_rows, L->d_tile_e,
-					   tiles, L->d_rec, L->d_hs, L->d_ypart, (int)T,
+					   tiles, L->d_rec, L->d_h, L->d_ypart, (int)T,
 					   (int)L->topk, (int)L->E, (int)L->EI, s),
 		     "grouped K-quant products");
 		LCHK(moe_launch_combine(L->d_ypart, w, d_out, (int)T, (int)L->topk, (int)L->E, 1, s),

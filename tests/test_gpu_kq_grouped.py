@@ -49,3 +49,22 @@ def test_gpu_kq_grouped_tiles_vs_oracle(name):
             assert np.array_equal(bits(out), bits(out_p)) and np.array_equal(ids, ids_p)
     finally:
         M.free()
+
+
+def test_gpu_kq_grouped_after_a_larger_reservation():
+    """Scratch reserved past the grouped products' limit: the same bits as
+    the oracle on both sides of it, from the one h buffer."""
+    wt, E, EI, NE, K = Q4K | Q6K << 8, 256, 256, 16, 8
+    lw = hipmoe.synth_layer(SEED, 12, wt, E, EI, NE, 0.02, None)
+    M = hipmoe.MoeLayer.from_synth(lw, K, False)
+    try:
+        assert hipmoe.lib().hip_moe_reserve(M.h, 36000) == 1
+        for T in (301, 3, 45):
+            x = hipmoe.synth_input(SEED, 0x9620 + T, T, E)
+            print(f"kq grouped after a reservation, T={T}", flush=True)
+            out, ids, w = M.ffn(x)
+            oout, oids, ow, _, _ = oracle.moe_ffn(x, lw, K, False, None)
+            assert np.array_equal(ids, oids) and np.array_equal(bits(w), bits(ow))
+            assert np.array_equal(bits(out), bits(oout))
+    finally:
+        M.free()

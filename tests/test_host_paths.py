@@ -1,0 +1,94 @@
+"""The host side of libhip_moe.so (dispatch, scratch, allocations that fail)
+on the CPU: the built library over tests/native/fake_hip.c, which logs kernel
+launches instead of running them.  Each case is a process of its own, since
+the fake runtime has to be loaded before the library."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from common import HERE, REPO
+
+PRELUDE = f"""
+import ctypes as C, sys
+F = C.CDLL({os.path.join(HERE, "native", "libfake_hip.so")!r}, mode=C.RTLD_GLOBAL)
+sys.path[:0] = [{os.path.join(REPO, "llm.c_amd")!r}]
+import numpy as np
+import hiplm, hipmoe
+for f in (F.fake_log, F.fake_sizes):
+    f.restype = C.c_char_p
+for f in (F.fake_fail_size, F.fake_fail_host):
+    f.argtypes = [C.c_size_t]
+F.fake_host_allocs.restype = C.c_size_t
+KQ = hipmoe.Q4_K | hipmoe.Q6_K << 8
+
+def layer(wt, E, EI, NE, K):
+    # byte 0 everywhere: valid blocks of any type
+    gt, dt = hipmoe.wtypes(wt)
+    gate = np.zeros((NE, EI * hipmoe.row_bytes(gt, E)), np.uint8)
+    down = np.zeros((NE, E * hipmoe.row_bytes(dt, EI)), np.uint8)
+    return hipmoe.MoeLayer(np.zeros((NE, E), np.float32), gate, gate, down, wt, E, EI, NE, K, 0)
+
+def kernels(call):
+    F.fake_log()
+    call()
+    return F.fake_log().decode()
+
+def dev_call(L, T):
+    # the pointers are handed on, never read
+    return kernels(lambda: L.ffn_dev(4096, 4096, T))
+"""
+
+
+def on_fake(body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], cwd=REPO,
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("reserve", (2000, 65535))
+def test_kq_grouped_whatever_was_reserved(reserve):
+    """The grouped K-quant products take a 301-token call on a layer whose
+    scratch was grown past the largest call they hold (about 34,800 tokens
+    here)."""
+    on_fake(f"""
+    L = layer(KQ, 256, 256, 16, 8)
+    hipmoe.lib().hip_moe_reserve(L.h, {reserve})
+    assert "k_kq_mm" in dev_call(L, 301)
+    assert "k_kq_mm" in dev_call(L, 34000)
+    assert "k_kq_mm" not in dev_call(L, 36000)
+    assert "k_kq_mm" in dev_call(L, 300)
+    """)
+
+
+def test_kq_grouped_shares_the_per_pair_scratch():
+    """One h buffer serves the per-pair and the grouped products."""
+    on_fake("""
+    L = layer(KQ, 256, 1024, 16, 8)
+    F.fake_sizes()
+    hipmoe.lib().hip_moe_reserve(L.h, 2000)
+    h = 2000 * 8 * 1024 * 4
+    big = [int(n) for n in F.fake_sizes().split() if int(n) >= h]
+    assert len(big) == 1 and big[0] < 1.05 * h, big
+    """)
+
+
+@pytest.mark.parametrize("which", ("h", "rows", "tiles", "records"))
+def test_kq_call_survives_a_failed_grouped_allocation(which):
+    """Without memory for the grouped products a call takes the per-pair
+    ones, as it did before there were others; with it again, later growth
+    brings them back."""
+    on_fake(f"""
+    L = layer(KQ, 256, 256, 16, 8)
+    T, K = 301, 8
+    tiles = (T * K + 31) // 32 + 16
+    F.fake_fail_size(dict(h=tiles * 32 * 256 * 4, rows=tiles * 32 * 4, tiles=(tiles + 1) * 4,
+                          records=T * 548)[{which!r}])
+    for _ in range(2):
+        got = dev_call(L, T)
+        assert "k_kq_mm" not in got and "k_kq_down" in got, got
+    F.fake_fail_size(0)
+    assert "k_kq_mm" in dev_call(L, 2 * T) and "k_kq_mm" in dev_call(L, T)
+    """)
