@@ -213,6 +213,11 @@ int hip_moe_expert_ffn_dev(hip_moe_layer *L, size_t expert, const float *d_x,
  * weights) is bit-identical on every path; outputs agree with the reference
  * within 1e-3 relative L2 (fp32 paths: ~1e-6; GROUPED: ~5e-4 from f16
  * operands).
+ * K-quant experts have the same outputs on every path, the reference's bit
+ * for bit: DECODE two launches (T*k <= 64), GEMV the per-pair products,
+ * GROUPED the same products with the pairs sorted by expert, which AUTO takes
+ * where the pairs past one per expert would re-read 40 MB of weights and
+ * which cannot be forced.
  */
 #define HIP_MOE_PATH_AUTO 0
 #define HIP_MOE_PATH_DECODE 1

@@ -408,6 +408,13 @@ static size_t kq_grouped_most(const hip_moe_layer *L)
 	return a < b ? a : b;
 }
 
+/* whether a call of T tokens takes them: with the scratch there is, or the
+ * one that the call makes */
+static int kq_grouped(const hip_moe_layer *L, size_t T)
+{
+	return kq_grouped_worth(L, T) && T <= (T > L->cap_T ? kq_grouped_most(L) : L->kq_T);
+}
+
 /* their buffers for T tokens, with one h for the P pairs of the other
  * kernels and their padded rows; without the memory none (a call then takes
  * the other kernels) */
@@ -737,8 +744,9 @@ int hip_moe_route_dev(hip_moe_layer *L, const float *d_x, size_t T,
 static int choose_path(const hip_moe_layer *L, size_t T)
 {
 	/* K-quant experts: two launches (routing and gate/up, then down and
-	 * combine) for a decode-sized call, else the per-pair products of
-	 * kq_moe.hip */
+	 * combine) for a decode-sized call, the grouped products of
+	 * kq_grouped.hip once the pairs re-read enough weights, else the
+	 * per-pair products of kq_moe.hip */
 	if (L->kq) {
 		const int kdec = L->fused_grid > 0 &&
 				 moe_kq_decode_supported(L->wtype, L->E, L->EI, L->NE, T, L->topk);
@@ -750,6 +758,8 @@ static int choose_path(const hip_moe_layer *L, size_t T)
 		case HIP_MOE_PATH_GROUPED:
 			return 0;
 		default:
+			if (kq_grouped(L, T))
+				return HIP_MOE_PATH_GROUPED;
 			return kdec ? HIP_MOE_PATH_DECODE : HIP_MOE_PATH_GEMV;
 		}
 	}
@@ -874,7 +884,7 @@ int hip_moe_ffn_dev(hip_moe_layer *L, const float *d_x, float *d_out, size_t T,
 		set_err("ffn: the requested path does not apply to this layer and T=%zu", T);
 		return 0;
 	}
-	if (L->kq && L->path == HIP_MOE_PATH_AUTO && T <= L->kq_T && kq_grouped_worth(L, T)) {
+	if (path == HIP_MOE_PATH_GROUPED && L->kq) {
 		const int tiles = (int)kq_tiles(L, (size_t)P);
 		if (!route(L, d_x, T, d_router_bias, L->d_logits, NULL, ids, w, NULL, s))
 			return 0;

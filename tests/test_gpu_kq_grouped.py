@@ -38,7 +38,9 @@ def test_gpu_kq_grouped_tiles_vs_oracle(name):
             x[T // 2] = 0.0  # an all-zero token: every Q8_K scale 0
             x[0, :256] *= 1e6
             M.set_path(hipmoe.PATH_AUTO)
+            assert M.path_for(T) == hipmoe.PATH_GROUPED
             out, ids, w = M.ffn(x)
+            assert M.path_for(T) == hipmoe.PATH_GROUPED
             M.set_path(hipmoe.PATH_GEMV)
             out_p, ids_p, w_p = M.ffn(x)
             oout, oids, ow, _, _ = oracle.moe_ffn(x, lw, K, bool(renorm), None)

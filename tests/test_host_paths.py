@@ -92,3 +92,30 @@ def test_kq_call_survives_a_failed_grouped_allocation(which):
     F.fake_fail_size(0)
     assert "k_kq_mm" in dev_call(L, 2 * T) and "k_kq_mm" in dev_call(L, T)
     """)
+
+
+@pytest.mark.parametrize("wt,E,EI,NE,K", (("KQ", 2048, 1024, 64, 8), ("KQ", 4096, 14336, 8, 2),
+                                          ("hipmoe.Q6_K", 1024, 512, 8, 2),
+                                          ("hipmoe.Q4_0", 2048, 1024, 64, 8)))
+def test_path_for_names_the_kernels_of_the_call(wt, E, EI, NE, K):
+    """hip_moe_path_for, asked before and after the scratch holds the call,
+    against the kernels the call launches, forced and not."""
+    on_fake(f"""
+    L = layer({wt}, {E}, {EI}, {NE}, {K})
+    of = dict(k_moe_decode=1, k_kq_route_gateup=1, k_gateup=2, k_kq_gateup=2, k_pf_gateup=3,
+              k_pf_gateup_v=3, k_kq_mm=3)
+    # mangled: the name behind its length
+    names = {{f"{{len(n)}}{{n}}": p for n, p in of.items()}}
+    seen = set()
+    for path in (0, 2):
+        L.set_path(path)
+        for T in (1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 16, 33, 64, 301, 7, 1):
+            said = L.path_for(T)
+            got = dev_call(L, T)
+            took = {{p for n, p in names.items() if n in got}}
+            assert took == {{said}} == {{L.path_for(T)}}, (path, T, said, took, got)
+            seen.add(said)
+    assert seen == {{1, 2, 3}}, seen
+    L.set_path(3)  # K-quants: AUTO alone takes the grouped products
+    assert L.path_for(301) == (0 if L.wtype != hipmoe.Q4_0 else 3)
+    """)
