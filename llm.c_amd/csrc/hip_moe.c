@@ -71,7 +71,7 @@ struct hip_moe_layer {
 	uint32_t *d_ids_io;
 	float *d_w_io;
 	/* pinned staging of host calls of a few tokens: x and the bias,
-	 * then out, ids, weights and the error word */
+	 * then out, ids, weights and the error word; NULL: they copy */
 	uint8_t *h_io;
 };
 
@@ -204,6 +204,35 @@ static int upload_down(hip_moe_layer *L, size_t e, const uint8_t *src, uint8_t *
 	return 1;
 fail:
 	return 0;
+}
+
+/* bytes of x of a host call that goes through the pinned staging: a few
+ * tokens, whose copies are all latency (more bytes are worth the copy
+ * engines) */
+#define IO_PINNED ((size_t)128 << 10)
+
+static size_t io_pinned_T(const hip_moe_layer *L)
+{
+	return IO_PINNED / (L->E * sizeof(float));
+}
+
+/* its words before the results: x and the bias */
+static size_t io_pinned_in(const hip_moe_layer *L)
+{
+	return io_pinned_T(L) * L->E + L->NE;
+}
+
+/* with the layer: page-locking takes about as long as the staging saves a
+ * call (40 us).  Without the memory host calls copy, as larger ones do. */
+static void io_pinned_alloc(hip_moe_layer *L)
+{
+	/* results, per token: out, ids, weights; and the error word */
+	const size_t words = io_pinned_in(L) + io_pinned_T(L) * (L->E + 2 * L->topk) + 1;
+	if (hipHostMalloc((void **)&L->h_io, words * sizeof(float), hipHostMallocPortable) !=
+	    hipSuccess) {
+		(void)hipGetLastError(); /* the launches check it */
+		L->h_io = NULL;
+	}
 }
 
 void hip_moe_free(hip_moe_layer *L)
@@ -363,6 +392,7 @@ hip_moe_layer *hip_moe_upload_typed(const float *gate_inp, const void *const *ga
 			goto fail;
 	}
 	free(stage);
+	io_pinned_alloc(L);
 	return L;
 fail:
 	free(stage);
@@ -1023,11 +1053,6 @@ fail:
 	return 0;
 }
 
-/* bytes of x of a host call that goes through the pinned staging: a few
- * tokens, whose copies are all latency (more bytes are worth the copy
- * engines) */
-#define IO_PINNED ((size_t)128 << 10)
-
 /*
  * A host call of a few tokens: x and the bias go through pinned memory that
  * one launch reads, and the results and the error word come back by one
@@ -1037,20 +1062,11 @@ fail:
 static int ffn_pinned(hip_moe_layer *L, const float *x, float *out, size_t T,
 		      const float *router_bias, uint32_t *ids_out, float *w_out)
 {
-	const size_t most = IO_PINNED / (L->E * sizeof(float)), P = T * L->topk;
-	if (T > most)
+	const size_t most = io_pinned_T(L), P = T * L->topk;
+	if (T > most || !L->h_io)
 		return -1;
-	/* per token: x, out, ids, weights; the bias and the error word */
-	const size_t in = most * L->E + L->NE, res = most * (L->E + 2 * L->topk) + 1;
-	if (!L->h_io) {
-		if (hipHostMalloc((void **)&L->h_io, (in + res) * sizeof(float),
-				  hipHostMallocPortable) != hipSuccess) {
-			L->h_io = NULL;
-			return -1;
-		}
-	}
 	hipStream_t s = L->stream;
-	float *hx = (float *)L->h_io, *hb = hx + most * L->E, *ho = hx + in;
+	float *hx = (float *)L->h_io, *hb = hx + most * L->E, *ho = hx + io_pinned_in(L);
 	uint32_t *hi = (uint32_t *)(ho + T * L->E), *he = hi + 2 * P;
 	memcpy(hx, x, T * L->E * sizeof(float));
 	if (router_bias)

@@ -119,3 +119,24 @@ def test_path_for_names_the_kernels_of_the_call(wt, E, EI, NE, K):
     L.set_path(3)  # K-quants: AUTO alone takes the grouped products
     assert L.path_for(301) == (0 if L.wtype != hipmoe.Q4_0 else 3)
     """)
+
+
+def test_first_host_call_locks_no_memory():
+    """The pinned staging of hip_moe_ffn is made with the layer."""
+    on_fake("""
+    L = layer(hipmoe.Q8_0, 2048, 1024, 8, 2)
+    n = F.fake_host_allocs()
+    got = kernels(lambda: L.ffn(np.zeros((1, 2048), np.float32)))
+    assert "k_copy_segs" in got and F.fake_host_allocs() == n, (got, n)
+    """)
+
+
+def test_host_call_without_page_locked_memory():
+    """A layer that got none takes the copies, every call of it."""
+    on_fake("""
+    F.fake_fail_host(1)
+    L = layer(hipmoe.Q8_0, 2048, 1024, 8, 2)
+    for _ in range(2):
+        got = kernels(lambda: L.ffn(np.zeros((1, 2048), np.float32)))
+        assert "k_copy_segs" not in got and "k_moe_decode" in got, got
+    """)
