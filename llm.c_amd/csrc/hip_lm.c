@@ -85,8 +85,9 @@ struct hip_lm {
 	unsigned graph_gen; /* the MoE layers' scratch generation the graphs name */
 	unsigned path_gen;  /* forced MoE path changes (hip_lm_set_moe_path) */
 	hipEvent_t ev0, ev1;
-	/* pinned: lm_launch_report's words (16), then a row of logits */
-	int *h_io;
+	/* lm_launch_report's words (16), then a row of logits; pinned unless
+	 * there was no such memory (the words are then read one by one) */
+	int *h_io, io_pinned;
 
 	/* prefill: a prompt of up to pf_cap rows in one forward, rows [T][.] */
 	size_t pf_cap, pf_heads; /* rows, and sequences whose last rows take the lm_head */
@@ -230,6 +231,25 @@ static void free_prefill(hip_lm *M)
 	M->pf_heads = 0;
 }
 
+/* host memory that copies and, if *pinned, kernels write */
+static int *host_words(size_t bytes, int *pinned)
+{
+	int *p = NULL;
+	*pinned = hipHostMalloc((void **)&p, bytes, hipHostMallocPortable) == hipSuccess;
+	if (*pinned)
+		return p;
+	(void)hipGetLastError(); /* the launches check it */
+	return malloc(bytes);
+}
+
+static void host_words_free(int *p, int pinned)
+{
+	if (pinned)
+		hipHostFree(p);
+	else
+		free(p);
+}
+
 void hip_lm_free(hip_lm *M)
 {
 	if (!M)
@@ -262,8 +282,7 @@ void hip_lm_free(hip_lm *M)
 			M->d_st, M->d_prompt, M->d_tokens};
 	for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
 		hipFree(bufs[i]);
-	if (M->h_io)
-		hipHostFree(M->h_io);
+	host_words_free(M->h_io, M->io_pinned);
 	if (M->ev0)
 		hipEventDestroy(M->ev0);
 	if (M->ev1)
@@ -414,8 +433,11 @@ hip_lm *hip_lm_upload(const hip_lm_desc *d)
 
 	HIPCHK(hipGetDevice(&M->device), "hipGetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&M->stream, hipStreamNonBlocking), "hipStreamCreate");
-	HIPCHK(hipHostMalloc((void **)&M->h_io, (16 + M->V) * sizeof(float),
-			     hipHostMallocPortable), "hipHostMalloc");
+	M->h_io = host_words((16 + M->V) * sizeof(float), &M->io_pinned);
+	if (!M->h_io) {
+		lm_err("lm_upload: out of host memory");
+		goto fail;
+	}
 	HIPCHK(hipEventCreate(&M->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&M->ev1), "hipEventCreate");
 
@@ -859,7 +881,7 @@ static int enqueue_report(const hip_lm *M, const LmState *st, const int *btok, s
 static int check_errors(hip_lm *M, const char *what)
 {
 	int err = 0;
-	if (enqueue_report(M, M->d_st, NULL, 0, M->h_io, M->stream)) {
+	if (M->io_pinned && enqueue_report(M, M->d_st, NULL, 0, M->h_io, M->stream)) {
 		HIPCHK(hipStreamSynchronize(M->stream), "synchronize");
 		if (!M->h_io[0] && !M->h_io[1])
 			return 1;
@@ -886,7 +908,7 @@ fail:
 	return 0;
 }
 
-/* the pinned row of logits */
+/* the host's row of logits */
 static float *h_logits(const hip_lm *M)
 {
 	return (float *)(M->h_io + 16);
@@ -1306,8 +1328,8 @@ struct hip_lm_batch {
 	hipGraphExec_t *g_body, *g_head;
 	unsigned graph_gen; /* the MoE layers' scratch generation the graphs name */
 	hipEvent_t ev0, ev1;
-	int *h_io;          /* pinned: lm_launch_report's words for S sequences */
-	float *h_logits;    /* pinned [S][V], NULL past BATCH_PINNED bytes */
+	int *h_io, io_pinned; /* lm_launch_report's words for S sequences */
+	float *h_logits;    /* pinned [S][V], NULL past BATCH_PINNED bytes or without such memory */
 };
 
 #define BATCH_PINNED ((size_t)16 << 20)
@@ -1340,8 +1362,7 @@ void hip_lm_batch_free(hip_lm_batch *B)
 			B->d_prompt, B->d_tokens, B->d_split};
 	for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
 		hipFree(bufs[i]);
-	if (B->h_io)
-		hipHostFree(B->h_io);
+	host_words_free(B->h_io, B->io_pinned);
 	if (B->h_logits)
 		hipHostFree(B->h_logits);
 	if (B->ev0)
@@ -1383,12 +1404,17 @@ hip_lm_batch *hip_lm_batch_new(hip_lm *M, size_t nseq)
 	const size_t part = S * M->H * (size_t)M->nch * (LM_HLEN + 2) * sizeof(uint64_t);
 	HIPCHK(hipSetDevice(M->device), "hipSetDevice");
 	HIPCHK(hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking), "hipStreamCreate");
-	HIPCHK(hipHostMalloc((void **)&B->h_io, (LM_REPORT_WORDS + S) * sizeof(int),
-			     hipHostMallocPortable), "hipHostMalloc");
-	if (S * M->V * sizeof(float) <= BATCH_PINNED)
-		HIPCHK(hipHostMalloc((void **)&B->h_logits, S * M->V * sizeof(float),
-				     hipHostMallocPortable),
-		       "hipHostMalloc");
+	B->h_io = host_words((LM_REPORT_WORDS + S) * sizeof(int), &B->io_pinned);
+	if (!B->h_io) {
+		lm_err("lm_batch_new: out of host memory");
+		goto fail;
+	}
+	if (S * M->V * sizeof(float) <= BATCH_PINNED &&
+	    hipHostMalloc((void **)&B->h_logits, S * M->V * sizeof(float), hipHostMallocPortable) !=
+		    hipSuccess) {
+		(void)hipGetLastError(); /* the launches check it */
+		B->h_logits = NULL;
+	}
 	HIPCHK(hipEventCreate(&B->ev0), "hipEventCreate");
 	HIPCHK(hipEventCreate(&B->ev1), "hipEventCreate");
 	HIPCHK(hipMalloc((void **)&B->d_kc, cache), "hipMalloc(batch k caches)");
@@ -1587,7 +1613,7 @@ fail:
 static int batch_errors(hip_lm_batch *B, const char *what)
 {
 	int err = 0;
-	if (enqueue_report(B->M, B->d_st, B->d_btok, B->S, B->h_io, B->stream)) {
+	if (B->io_pinned && enqueue_report(B->M, B->d_st, B->d_btok, B->S, B->h_io, B->stream)) {
 		HIPCHK(hipStreamSynchronize(B->stream), "synchronize");
 		if (!B->h_io[0] && !B->h_io[1])
 			return 1;

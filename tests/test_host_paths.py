@@ -140,3 +140,26 @@ def test_host_call_without_page_locked_memory():
         got = kernels(lambda: L.ffn(np.zeros((1, 2048), np.float32)))
         assert "k_copy_segs" not in got and "k_moe_decode" in got, got
     """)
+
+
+TINY = "hiplm.synth_olmoe(1, 1, 256, 2, 256, 4, 2, 256, hipmoe.Q8_0)"
+
+
+def test_model_and_batch_without_page_locked_memory():
+    """Upload and every host call of a model work from plain host memory."""
+    on_fake(f"""
+    md = {TINY}
+    F.fake_fail_host(1)
+    M = hiplm.LmModel(md, 64)
+    ids = np.arange(5, dtype=np.int32)
+    M.prefill(ids)
+    M.decode(3)
+    M.reset()
+    assert len(M.generate(ids, 3)[0]) == 4
+    B = hiplm.LmBatch(M, 3)
+    B.decode(ids[:3])
+    B.reset()
+    B.generate(np.tile(ids, (3, 1)), 2)
+    B.free()
+    M.free()
+    """)
