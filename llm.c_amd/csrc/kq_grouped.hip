@@ -124,7 +124,6 @@ __device__ static inline half8_t km_op(u32 a, u32 b, u32 m, half2_t s, half2_t o
 template <int WT> struct kmw;
 
 template <> struct kmw<3> {
-	static constexpr int LOADS = 5;
 	u32x4 hd, q[4];
 	__device__ inline void load(const uint8_t *blk, int h)
 	{
@@ -145,7 +144,6 @@ template <> struct kmw<3> {
 };
 
 template <> struct kmw<5> {
-	static constexpr int LOADS = 8;
 	u32x4_a2 ql[4], qh[2], sc;
 	unsigned short d;
 	__device__ inline void load(const uint8_t *blk, int h)
@@ -408,9 +406,13 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 	for (int c = 0; c < NC; c++)
 		w[c].pin();
 	for (int sb = 0; sb < nb; sb++) {
-		/* super-block sb's records have landed: only the weights' loads,
-		 * issued after them, may be in flight (loads retire in order) */
-		wait_vm<NC * kmw<WT>::LOADS>();
+		/* super-block sb's records have landed once the first matrix's
+		 * weights have: those loads were issued after them, and loads
+		 * retire in order (the compiler waits for them here: a wait that
+		 * counted the loads behind the records would rest on how many
+		 * it makes of them) */
+		w[0].pin();
+		asm volatile("" ::: "memory");
 		__syncthreads(); /* every wave's share; the other buffer is free */
 		const int nx = min(sb + 1, nb - 1);
 		if (sb + 1 < nb)
@@ -421,7 +423,8 @@ __global__ __launch_bounds__(NW * WAVE, 2) void k_kq_mm(
 #pragma unroll
 		for (int c = 0; c < NC; c++) {
 			floatx16 S1, S2;
-			w[c].pin(); /* not ahead of the other matrix's loads */
+			if (c)
+				w[c].pin(); /* not ahead of the other matrix's loads */
 			km_mins<LR>(w[c], sa, m, h, yd, accm[c]);
 			__builtin_amdgcn_sched_barrier(0);
 			km_sums<LR>(w[c], sa, m, h, S1, S2);
