@@ -1381,6 +1381,8 @@ static size_t tok_lds(int K)
 static const void *lm_kernel(int kind, int wtype, int K)
 {
 	const int C = moe_lanes_per_row((size_t)K);
+	if (moe_kchunks((size_t)K) != 1)
+		return nullptr; /* a lane holds one segment of a row */
 #define LMK(WTT, CC)                                                                    \
 	if (wtype == WTT && C == CC)                                                    \
 		return kind == 0 ? (const void *)k_lm_qkv<WTT, CC>                       \

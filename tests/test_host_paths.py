@@ -163,3 +163,19 @@ def test_model_and_batch_without_page_locked_memory():
     B.free()
     M.free()
     """)
+
+
+@pytest.mark.parametrize("heads,ok", ((4, True), (6, False)))
+def test_model_refuses_head_rows_no_kernel_covers(heads, ok):
+    """The one-token products cover rows of 64 columns times a power of two
+    up to 64; heads * 128 = 768 would leave two thirds of a row out."""
+    on_fake(f"""
+    md = hiplm.synth_mixtral(1, 1, 512, {heads}, 2, 256, 4, 2, 256, hipmoe.Q4_0)
+    try:
+        hiplm.LmModel(md, 64)
+        ok = True
+    except hipmoe.HipMoeError as e:
+        assert "not supported" in str(e)
+        ok = False
+    assert ok == {ok}
+    """)
