@@ -307,7 +307,7 @@ static int product_ok(int t, size_t K)
 
 static int product_grid(int t, size_t K)
 {
-	return is_kq(t) ? moe_kq_grid(t, (int)K, 1) : moe_qgemv_grid(t, (int)K, 1);
+	return is_kq(t) ? moe_kq_grid(t, (int)K, 1) : moe_qgemv_grid(t, (int)K);
 }
 
 /* out[N] = add + x . W^T for one token (add NULL or [N]) in type t */
@@ -317,7 +317,7 @@ static int vec_product(int t, const uint8_t *W, int N, int K, const float *x, co
 	if (is_kq(t))
 		LCHK(moe_launch_kq_gemv(t, W, N, K, x, 1, add, 0, out, grid, s), "product");
 	else
-		LCHK(moe_launch_qgemv(t, W, N, K, x, 1, add, 0, out, grid, s), "product");
+		LCHK(moe_launch_qgemv(t, W, N, K, x, add, out, grid, s), "product");
 	return 1;
 }
 
@@ -950,11 +950,11 @@ static int ensure_prefill(hip_lm *M, size_t T, size_t nseq)
 	HIPCHK(hipMalloc((void **)&M->d_pf_qkv, T * NQKV * 4), "hipMalloc(prefill qkv)");
 	HIPCHK(hipMalloc((void **)&M->d_pf_q, T * M->EQ * 4), "hipMalloc(prefill q)");
 	HIPCHK(hipMalloc((void **)&M->d_pf_attn, T * M->EQ * 4), "hipMalloc(prefill attn)");
-	{ /* the partial sums of the largest of the three products: q/k/v and
-	   * output over T rows, the lm_head over the nseq last rows */
-		size_t wb = moe_qmm_work_bytes((int)T, (int)NQKV, (int)E);
-		const size_t w2 = moe_qmm_work_bytes((int)T, (int)E, (int)M->EQ);
-		const size_t w3 = moe_qmm_work_bytes((int)nseq, (int)M->V, (int)E);
+	{ /* the partial sums of the largest of the three products that has some:
+	   * q/k/v and output over up to T rows, the lm_head over the last rows */
+		size_t wb = moe_qmm_work_most((int)T, (int)NQKV, (int)E);
+		const size_t w2 = moe_qmm_work_most((int)T, (int)E, (int)M->EQ);
+		const size_t w3 = moe_qmm_work_most((int)nseq, (int)M->V, (int)E);
 		wb = wb > w2 ? wb : w2;
 		wb = wb > w3 ? wb : w3;
 		if (wb)
@@ -971,20 +971,16 @@ fail:
 	return 0;
 }
 
-/* out[T][N] = add + x[T][K] . W^T (add NULL or [T][N]): the matrix cores
- * where K suits them, else the per-token product */
+/* out[T][N] = add + x[T][K] . W^T (add NULL or [T][N]) on the matrix cores */
 static int rows_product(hip_lm *M, const uint8_t *W, int N, int K, const float *x, int T,
 			const float *add, float *out, hipStream_t s)
 {
 	const int wt = M->wtype;
-	if (moe_qmm_supported(wt, K) && moe_qmm_tile_better(N, T))
+	if (moe_qmm_tile_better(N, T))
 		LCHK(moe_launch_qmm_tile(wt, W, N, K, x, T, add, add != NULL, out, s),
 		     "prefill product");
-	else if (moe_qmm_supported(wt, K))
-		LCHK(moe_launch_qmm(wt, W, N, K, x, T, add, add != NULL, out, M->d_pf_split, s),
-		     "prefill product");
 	else
-		LCHK(moe_launch_qgemv(wt, W, N, K, x, T, add, add != NULL, out, 0, s),
+		LCHK(moe_launch_qmm(wt, W, N, K, x, T, add, add != NULL, out, M->d_pf_split, s),
 		     "prefill product");
 	return 1;
 }
@@ -1434,9 +1430,9 @@ hip_lm_batch *hip_lm_batch_new(hip_lm *M, size_t nseq)
 	HIPCHK(hipMalloc((void **)&B->d_cnt, S * M->H * sizeof(uint32_t)), "hipMalloc(counters)");
 	HIPCHK(hipMemset(B->d_cnt, 0, S * M->H * sizeof(uint32_t)), "clear counters");
 	{ /* the largest partial sums: the lm_head's or the q/k/v product's */
-		size_t wb = moe_qmm_work_bytes((int)S, (int)M->V, (int)E);
-		const size_t w2 = moe_qmm_work_bytes((int)S, (int)(M->EQ + 2 * M->EKV), (int)E);
-		const size_t w3 = moe_qmm_work_bytes((int)S, (int)E, (int)M->EQ);
+		size_t wb = moe_qmm_work_most((int)S, (int)M->V, (int)E);
+		const size_t w2 = moe_qmm_work_most((int)S, (int)(M->EQ + 2 * M->EKV), (int)E);
+		const size_t w3 = moe_qmm_work_most((int)S, (int)E, (int)M->EQ);
 		wb = wb > w2 ? wb : w2;
 		wb = wb > w3 ? wb : w3;
 		if (wb)
@@ -1494,21 +1490,16 @@ fail:
 	return 0;
 }
 
-/* out[S][N] = add + x[S][K] . W^T: on the matrix cores where K suits
- * them, else the per-token product */
+/* out[S][N] = add + x[S][K] . W^T on the matrix cores */
 static int batch_product(hip_lm_batch *B, const uint8_t *W, int N, int K, const float *x,
 			 const float *add, float *out)
 {
 	const int wt = B->M->wtype, S = (int)B->S;
-	if (moe_qmm_supported(wt, K) && moe_qmm_tile_better(N, S)) {
+	if (moe_qmm_tile_better(N, S))
 		LCHK(moe_launch_qmm_tile(wt, W, N, K, x, S, add, add != NULL, out, B->stream), "product");
-	} else if (moe_qmm_supported(wt, K)) {
+	else
 		LCHK(moe_launch_qmm(wt, W, N, K, x, S, add, add != NULL, out, B->d_split, B->stream),
 		     "product");
-	} else {
-		LCHK(moe_launch_qgemv(wt, W, N, K, x, S, add, add != NULL, out, 0, B->stream),
-		     "product");
-	}
 	return 1;
 }
 
@@ -1537,8 +1528,7 @@ static int batch_step(hip_lm_batch *B, int head, int nact)
 		 * product leaves partial sums, one launch adds them (the reduce's
 		 * order), adds h0 and normalises */
 		const int EQ = (int)M->EQ;
-		if (moe_qmm_supported(wt, EQ) && moe_qmm_stretches(EQ) > 1 &&
-		    !moe_qmm_tile_better(E, S)) {
+		if (moe_qmm_stretches(EQ) > 1 && !moe_qmm_tile_better(E, S)) {
 			LCHK(moe_launch_qmm_parts(wt, y->wo, E, EQ, B->d_attn, S, B->d_split, s),
 			     "output product");
 			LCHK(lm_launch_norm_parts(S, E, B->d_split, moe_qmm_stretches(EQ), (size_t)S * E,

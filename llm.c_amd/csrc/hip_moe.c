@@ -1158,12 +1158,11 @@ struct hip_moe_qmat {
 	size_t N, K, bytes;
 	uint8_t *d_w;       /* the GGUF blocks, row-major, unchanged */
 	hipStream_t stream; /* the device's shared library stream */
-	int grid1, grid;    /* workgroups for T == 1 and T > 1 (moe_qgemv_grid) */
+	int grid1, grid;    /* workgroups for T == 1 and (K-quants) T > 1 */
 	/* the partial sums of the matrix-core product (T > 1), for up to
 	 * split_T tokens; calls that overlap on one matrix race on them */
 	void *d_split;
 	size_t split_T;
-	int qmm;            /* K suits the matrix-core product */
 	/* staging for the host-pointer entry point */
 	size_t cap_T;
 	float *d_x, *d_add, *d_out;
@@ -1181,7 +1180,7 @@ static int qmat_split_alloc(hip_moe_qmat *W, size_t T)
 	hipFree(W->d_split);
 	W->d_split = NULL;
 	W->split_T = 0;
-	const size_t wb = moe_qmm_work_bytes((int)T, (int)W->N, (int)W->K);
+	const size_t wb = moe_qmm_work_most((int)T, (int)W->N, (int)W->K);
 	if (wb)
 		HIPCHK(hipMalloc(&W->d_split, wb), "hipMalloc(qmat partial sums)");
 	W->split_T = T;
@@ -1241,12 +1240,10 @@ hip_moe_qmat *hip_moe_qmat_upload(const void *qdata, int wtype, size_t N, size_t
 		W->grid1 = moe_kq_grid(wtype, (int)K, 1);
 		W->grid = moe_kq_grid(wtype, (int)K, 8);
 	} else {
-		W->grid1 = moe_qgemv_grid(wtype, (int)K, 1);
-		W->grid = moe_qgemv_grid(wtype, (int)K, 0);
+		W->grid1 = moe_qgemv_grid(wtype, (int)K);
+		if (!qmat_split_alloc(W, QMAT_SPLIT_T))
+			goto fail;
 	}
-	W->qmm = !is_kquant(wtype) && moe_qmm_supported(wtype, (int)K);
-	if (W->qmm && !qmat_split_alloc(W, QMAT_SPLIT_T))
-		goto fail;
 	/* the K-quant loads read up to MOE_KQ_SLACK bytes past the last block */
 	HIPCHK(hipMalloc((void **)&W->d_w, W->bytes + MOE_KQ_SLACK), "hipMalloc(qmat)");
 	HIPCHK(hipMemset(W->d_w + W->bytes, 0, MOE_KQ_SLACK), "clear qmat slack");
@@ -1294,19 +1291,18 @@ int hip_moe_qmat_mul_dev(const hip_moe_qmat *W, const float *d_x, size_t T,
 		LCHK(moe_launch_kq_gemv(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 					add_len == T * W->N, d_out, T == 1 ? W->grid1 : W->grid, s),
 		     "kq_gemv");
-	} else if (T > 1 && W->qmm &&
-		   (T > W->split_T || moe_qmm_tile_better((int)W->N, (int)T))) {
+	} else if (T == 1) {
+		LCHK(moe_launch_qgemv(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, d_add, d_out,
+				      W->grid1, s), "qgemv");
+	} else if (T > W->split_T || moe_qmm_tile_better((int)W->N, (int)T)) {
 		/* several tokens: on the matrix cores, at fp32 accuracy; in tiles of
 		 * tokens where those are faster or the split buffer holds fewer */
 		LCHK(moe_launch_qmm_tile(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 					 add_len == T * W->N, d_out, s), "qmm_tile");
-	} else if (T > 1 && W->qmm) {
+	} else {
 		LCHK(moe_launch_qmm(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
 				    add_len == T * W->N, d_out, W->d_split, s), "qmm");
-	} else
-		LCHK(moe_launch_qgemv(W->wtype, W->d_w, (int)W->N, (int)W->K, d_x, (int)T, d_add,
-				      add_len == T * W->N, d_out, T == 1 ? W->grid1 : W->grid, s),
-		     "qgemv");
+	}
 	return 1;
 }
 
@@ -1336,7 +1332,7 @@ int hip_moe_qmat_mul(hip_moe_qmat *W, const float *x, size_t T, const float *add
 		W->cap_T = T;
 	}
 	/* the host entry point may allocate */
-	if (W->qmm && T > W->split_T && !moe_qmm_tile_better((int)W->N, (int)T)) {
+	if (!is_kquant(W->wtype) && T > W->split_T && !moe_qmm_tile_better((int)W->N, (int)T)) {
 		/* device-pointer calls on any stream may still read the old buffer */
 		HIPCHK(hipDeviceSynchronize(), "synchronize");
 		if (!qmat_split_alloc(W, T))

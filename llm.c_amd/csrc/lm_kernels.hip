@@ -277,7 +277,7 @@ void k_lm_qkv(const uint8_t *__restrict__ W, size_t rb, int N, int K, const floa
 	const uint8_t *emb =
 		a ? nullptr : wte + (size_t)step_token(st, prompt) * (size_t)(K / 32) * BB;
 	stage_norm<WT>(sx, red, K, a, b, emb, w, blockIdx.x == 0 ? h_out : nullptr);
-	qgemv_body<WT, C, true, true>(sx, W, rb, N, K, nullptr, 1, 1, nullptr, 0, out);
+	qgemv_body<WT, C, true>(sx, W, rb, N, K, nullptr, nullptr, out);
 }
 
 /* ---------------------------------------------------------------------- */
@@ -676,12 +676,12 @@ void k_lm_oproj(const uint8_t *__restrict__ W, size_t rb, int N, int K,
 	extern __shared__ __attribute__((aligned(16))) float sx[];
 	__shared__ float red[LM_NT / WAVE];
 	if (!x_out) {
-		qgemv_body<WT, C, true>(sx, W, rb, N, K, x, 1, 1, add, 0, out, QgNoHook{});
+		qgemv_body<WT, C>(sx, W, rb, N, K, x, add, out);
 		return;
 	}
 	const u32 tag = lm_tag(st, layer);
 	auto hook = [=](int row, float r) { st_dev_u64(&rows_t[row], tagged(tag, r)); };
-	qgemv_body<WT, C, true>(sx, W, rb, N, K, x, 1, 1, add, 0, out, hook);
+	qgemv_body<WT, C, false>(sx, W, rb, N, K, x, add, out, hook);
 	/* workgroup 0 normalises, polling the rows as they land: the host sizes
 	 * the grid to be resident at once, so every row comes (counting the
 	 * workgroups in at device counters put 2-3 us of atomics behind the
@@ -757,7 +757,7 @@ void k_lm_head(const uint8_t *__restrict__ W, size_t rb, int N, int K, const flo
 	float bv = -INFINITY;
 	int bi = 0x7fffffff;
 	auto hook = [&](int row, float r) { better(bv, bi, r, row); };
-	qgemv_body<WT, C, true, true>(sx, W, rb, N, K, nullptr, 1, 1, nullptr, 0, out, hook);
+	qgemv_body<WT, C, true>(sx, W, rb, N, K, nullptr, nullptr, out, hook);
 	for (int o = WAVE / 2; o > 0; o >>= 1)
 		better(bv, bi, __shfl_xor(bv, o, WAVE), __shfl_xor(bi, o, WAVE));
 	const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;

@@ -58,21 +58,22 @@ int moe_launch_down(int wtype, const uint8_t *down, size_t expert_stride,
                     const uint32_t *ids, int fixed_e, const float *h,
                     float *ypart, size_t ypart_cap, int P, int E, int EI, int *kchunks,
                     void *stream);
-/* out[t][j] = (add ? add[add_rows ? t*N + j : j] : 0) + dot(x[t], W row j),
- * W of N rows of K columns in Q8_0 (wtype 1) or Q4_0 (2) blocks; K/64 a
- * power of two 4..64; x 16-byte aligned (moe_qgemv.hip).  nwg workgroups
- * (moe_qgemv_grid; <= 0: a fixed default). */
-int moe_launch_qgemv(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
-                     const float *add, int add_rows, float *out, int nwg, void *stream);
-/* workgroups the device holds at once for the (wtype, K, T == 1) instance */
-int moe_qgemv_grid(int wtype, int K, int one);
+/* out[j] = (add ? add[j] : 0) + dot(x, W row j) of one token, W of N rows of
+ * K columns in Q8_0 (wtype 1) or Q4_0 (2) blocks; K/64 a power of two 4..64;
+ * x 16-byte aligned (moe_qgemv.hip).  nwg workgroups (moe_qgemv_grid; <= 0: a
+ * fixed default). */
+int moe_launch_qgemv(int wtype, const uint8_t *W, int N, int K, const float *x,
+                     const float *add, float *out, int nwg, void *stream);
+/* workgroups the device holds at once for the (wtype, K) instance */
+int moe_qgemv_grid(int wtype, int K);
 
 /* the same product for several tokens on the matrix cores at fp32
  * accuracy (moe_qmm.hip): x [T][K] fp32, 16-byte aligned; K = 256, 512
- * or a multiple of 512 (moe_qmm_supported); work holds
- * moe_qmm_work_bytes(T, N, K) bytes (none for K <= 512) */
-int moe_qmm_supported(int wtype, int K);
+ * or a multiple of 512; work holds moe_qmm_work_bytes(T, N, K) bytes (none
+ * for K <= 512).  moe_qmm_work_most: the most that any product of up to T
+ * tokens needs which the tiles below do not take. */
 size_t moe_qmm_work_bytes(int T, int N, int K);
+size_t moe_qmm_work_most(int T, int N, int K);
 int moe_launch_qmm(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
                    const float *add, int add_rows, float *out, void *work, void *stream);
 /* the same product in tiles of 32 or 64 tokens, without scratch memory; K a

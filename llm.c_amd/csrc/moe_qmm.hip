@@ -666,7 +666,7 @@ static int qmm_pz(int K)
 	return K / 64 < QMM_PZ ? K / 64 : QMM_PZ;
 }
 
-extern "C" int moe_qmm_supported(int wtype, int K)
+static bool qmm_supported(int wtype, int K)
 {
 	return (wtype == 1 || wtype == 2) && K >= 256 && K % 256 == 0 &&
 	       (K <= 64 * QMM_PZ ? ((K / 256) & (K / 256 - 1)) == 0 : K % (64 * QMM_PZ) == 0);
@@ -692,7 +692,7 @@ static int launch_qmm(int wtype, const uint8_t *W, int N, int K, const float *x,
 		      const float *add, int add_rows, float *out, void *work, bool parts_only,
 		      void *stream)
 {
-	if (!moe_qmm_supported(wtype, K) || N < 1 || T < 1 || (size_t)T * N > 0xffffffffull)
+	if (!qmm_supported(wtype, K) || N < 1 || T < 1 || (size_t)T * N > 0xffffffffull)
 		return (int)hipErrorInvalidValue;
 	const int PZ = qmm_pz(K), KS = K / (64 * PZ);
 	if ((T + QMM_TOK - 1) / QMM_TOK > 65535 || (KS > 1 && !work) || (parts_only && KS < 2))
@@ -770,6 +770,13 @@ extern "C" int moe_qmm_tile_better(int N, int T)
 	return w > 228 * SMALL_ROUNDS(N, T) || w > 540 * WIDE_ROUNDS(N, T);
 }
 
+extern "C" size_t moe_qmm_work_most(int T, int N, int K)
+{
+	while (T > 0 && moe_qmm_tile_better(N, T))
+		T--;
+	return moe_qmm_work_bytes(T, N, K);
+}
+
 template <int WT, int NW, int TM>
 static hipError_t launch_tile(const uint8_t *W, size_t rb, int N, int K, const float *x, int T,
 			      const float *add, int add_rows, float *out, hipStream_t s)
@@ -786,7 +793,7 @@ static hipError_t launch_tile(const uint8_t *W, size_t rb, int N, int K, const f
 extern "C" int moe_launch_qmm_tile(int wtype, const uint8_t *W, int N, int K, const float *x, int T,
 				   const float *add, int add_rows, float *out, void *stream)
 {
-	if ((wtype != 1 && wtype != 2) || N < 1 || T < 1 || K < 128 || K % 128)
+	if (!qmm_supported(wtype, K) || N < 1 || T < 1)
 		return (int)hipErrorInvalidValue;
 	const size_t rb = (size_t)(K / 32) * (wtype == 1 ? 34 : 18);
 	hipStream_t s = (hipStream_t)stream;

@@ -646,7 +646,7 @@ def test_gpu_qmat_matrix_cores_vs_oracle(wt):
     scale applied in fp32): every K it takes (256 .. 4096), token counts
     that fill one tile, pad one (T = 3) and span three (T = 33), ragged N,
     held to the fp32 bar TIGHT against the oracle; T = 65 goes past the
-    split buffer of the device entry point (the per-token product) and
+    split buffer of the device entry point (the tiles) and
     through the host entry point (which grows it)."""
     H = hipmoe.hip()
     for K in (256, 512, 1024, 2048, 4096):

@@ -179,3 +179,31 @@ def test_model_refuses_head_rows_no_kernel_covers(heads, ok):
         ok = False
     assert ok == {ok}
     """)
+
+
+@pytest.mark.parametrize("N,K", ((300, 256), (2048, 2048), (6144, 2048), (4096, 4096), (32000, 4096)))
+def test_split_buffer_holds_what_the_few_token_form_writes(N, K):
+    """A matrix's partial sums: enough for every token count that takes the
+    form with partial sums, none where no count does; one token has its own
+    kernel, larger counts the tiles."""
+    on_fake(f"""
+    N, K, top = {N}, {K}, 64
+    lib = hipmoe.lib()
+    for f in (lib.moe_qmm_work_bytes, lib.moe_qmm_work_most):
+        f.restype = C.c_size_t
+    few = [t > 0 and not lib.moe_qmm_tile_better(N, t) for t in range(2001)]
+    for T in (2, 16, 40, 64, 333, 2000):
+        need = max(lib.moe_qmm_work_bytes(t, N, K) if few[t] else 0 for t in range(T + 1))
+        assert lib.moe_qmm_work_most(T, N, K) == need, T
+    F.fake_sizes()
+    W = hipmoe.QMat(np.zeros(N * hipmoe.row_bytes(hipmoe.Q4_0, K), np.uint8), hipmoe.Q4_0, N, K)
+    sizes = [int(n) for n in F.fake_sizes().split()]
+    weights = max(sizes)
+    split = [n for n in sizes if n != weights]
+    assert sum(split) == lib.moe_qmm_work_most(top, N, K), sizes
+    for T in (1, 2, 16, 17, 64, 65, 301):
+        got = kernels(lambda: W.mul_dev(4096, T, 4096))
+        want = "k_qgemv1" if T == 1 else "5k_qmmI" if few[T] and T <= top else "k_qmm_tile"
+        assert [n for n in ("k_qgemv", "5k_qmmI", "k_qmm_tile") if n in got] == \
+            [want.removesuffix("1")], (T, got)
+    """)
