@@ -50,9 +50,31 @@ def test_gpu_batch_of_more_sequences_than_one_launch_sets():
             got[S] = [B.decode(ids[:S, i]) for i in range(3)]
             B.free()
         for (n0, l0), (n1, l1) in zip(got[128], got[130]):
+            assert np.array_equal(n0, l0.argmax(1)) and np.array_equal(n1, l1.argmax(1))
             err = rel_l2(l1[:128], l0)
             print(f"batch of 130 against 128: {err:.2e}", flush=True)
             # the same products row by row; their sums may be split otherwise
             assert err <= 1e-5
+    finally:
+        M.free()
+
+
+def test_gpu_batch_of_more_logits_than_are_pinned():
+    """17 MB of logits a step are copied, 2 MB go through pinned memory:
+    the same rows, and each row's pick."""
+    md = hiplm.synth_olmoe(SEED, 1, 512, 4, 34000, 8, 2, 256, hipmoe.Q8_0, 0.1)
+    M = hiplm.LmModel(md, 32)
+    try:
+        ids = np.random.default_rng(SEED).integers(0, md["V"], (128, 2)).astype(np.int32)
+        got = {}
+        for S in (16, 128):
+            B = hiplm.LmBatch(M, S)
+            got[S] = [B.decode(ids[:S, i]) for i in range(2)]
+            B.free()
+        for (n0, l0), (n1, l1) in zip(got[16], got[128]):
+            assert np.array_equal(n0, l0.argmax(1)) and np.array_equal(n1, l1.argmax(1))
+            err = rel_l2(l1[:16], l0)
+            print(f"batch of 128 against 16: {err:.2e}", flush=True)
+            assert err <= 1e-5  # the same products; their sums may be split otherwise
     finally:
         M.free()

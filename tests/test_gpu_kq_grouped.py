@@ -70,3 +70,29 @@ def test_gpu_kq_grouped_after_a_larger_reservation():
             assert np.array_equal(bits(out), bits(oout))
     finally:
         M.free()
+
+
+@pytest.mark.parametrize("wt", (Q4K | Q6K << 8, Q6K | Q4K << 8))
+def test_gpu_kq_grouped_extreme_h_vs_oracle(wt):
+    """Tokens whose h overflows, is subnormal, or makes subnormal products
+    with the down weights: the matrix instructions' chains keep the bits of
+    the oracle's FMAs, and have NaN and infinities where it has."""
+    E, EI, NE, K, T = 512, 512, 4, 2, 120
+    lw = hipmoe.synth_layer(SEED, 13, wt, E, EI, NE, 0.02, None)
+    x = hipmoe.synth_input(SEED, 0x9630, T, E)
+    scale = np.float32([1, 1e25, 1e-19, 1e-21, 1e-17, 2e19])
+    x *= scale[np.arange(T) % scale.size][:, None]
+    M = hipmoe.MoeLayer.from_synth(lw, K, False)
+    try:
+        assert M.path_for(T) == hipmoe.PATH_GROUPED
+        out, _, _ = M.ffn(x)
+        want, _, _, _, _ = oracle.moe_ffn(x, lw, K, False, None)
+        small = np.abs(want[want != 0])
+        print(f"kq grouped extremes {wt:#x}: {np.isnan(want).sum()} NaN, {np.isinf(want).sum()} "
+              f"infinite, {(small < 2.0**-126).sum()} subnormal of {want.size}", flush=True)
+        assert np.isnan(want).any() and (small < 2.0**-126).any()
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(out), nan)
+        assert np.array_equal(bits(out)[~nan], bits(want)[~nan])
+    finally:
+        M.free()
