@@ -36,9 +36,10 @@
  * of vector_avx2.h:126-132 joins the eight tiles at the end.
  *
  * Measured (Q4_K gate/up, Q6_K down): 2048 x 1024, 64 experts top-8, 301
- * tokens: 3471 -> 280 us a layer against a workgroup per pair and 32 rows
- * (gate/up 930 -> 91, down 2608 -> 187 us); 4096 x 14336, 8 top-2, 200
- * tokens: 15762 -> 994 us (6361 -> 291, 9176 -> about 690).
+ * tokens: 3456 -> 282 us a layer against a workgroup per pair and 32 rows
+ * (under a profiler gate/up 930 -> 91, down 2608 -> 191 us); 4096 x 14336, 8
+ * top-2, 200 tokens: 15490 -> 988 us (under a profiler, a tenth slower: 6361 ->
+ * 315, 9176 -> 767).
  */
 #include "kq_device.h"
 #include "moe_internal.h"
@@ -343,8 +344,8 @@ __device__ static inline int km_item(int id, int items)
  * its last one is used.
  *
  * Bound: the VALU, of which the operands take about 2/3 (9 instructions per
- * 8 weights) and the fp32 steps 1/3, beside 34 MFMAs a matrix and super-block
- * (two waves a SIMD overlap them); for many-expert layers of few rows a tile
+ * 8 weights) and the fp32 steps 1/3, beside 17 (Q4_K: 16 and the minima's) or
+ * 32 (Q6_K) MFMAs a matrix and super-block (two waves a SIMD overlap them); for many-expert layers of few rows a tile
  * the weights' bytes come next.  32 rows a tile: 64 need 256 registers of
  * accumulators, and the experts of a prompt average 10 to 60 rows.
  */
@@ -546,11 +547,11 @@ __device__ static inline void kq_stage(const float4 (&v)[8], uint8_t *sa, float 
  * costs about as much as the operands of one wave's 32 columns.
  *
  * Bound: the VALU, which the MFMAs' cycles add to where they share a SIMD.
- * 4096 x 4096 Q4_K: 77 tokens 384 -> 42 us, 333 tokens 1771 -> 70 us against
- * the per-token product (whose groups of tokens re-read and re-unpack every
- * weight); Q6_K 390 -> 55 and 1772 -> 96 us; 4096 x 14336 Q4_K, 77 tokens:
- * 2132 -> 140 us.  With every wave quantizing and then multiplying: 47, 71,
- * 78, 115 and 154 us.
+ * Kernel times under a profiler, 4096 x 4096 Q4_K: 77 tokens 384 -> 42 us (the
+ * whole call 413 -> 44), 333 tokens 1771 -> 70 us against the per-token
+ * product (whose groups of tokens re-read and re-unpack every weight); Q6_K
+ * 390 -> 55 and 1772 -> 96 us; 4096 x 14336 Q4_K, 77 tokens: 2132 -> 140 us.
+ * With every wave quantizing and then multiplying: 47, 71, 78, 115 and 154 us.
  */
 template <int WT>
 __global__ __launch_bounds__(2 * KD_WAVES * WAVE, 4) void k_kq_dense(

@@ -203,8 +203,7 @@ __global__ __launch_bounds__(QMM_WAVES * WAVE) void k_qmm(
 	 * (block, group, token), the token fastest, so a wave's stores are 1 KB
 	 * contiguous (with the group fastest every lane of a wave hit the same
 	 * banks); all of a thread's loads go out before any is used (a loop
-	 * that waited for each made the staging eight round trips: 33 -> ? us
-	 * for the Mixtral q/k/v product of 16 tokens) */
+	 * that waited for each made the staging eight round trips) */
 	constexpr int IT = QMM_TOK * NB * 4 / (QMM_WAVES * WAVE); /* items per thread */
 	float v[IT][8];
 #pragma unroll
