@@ -61,7 +61,7 @@ typedef struct hip_lm_desc {
 	const float *const *attn_norm;                /* [E] */
 	const void *const *attn_q;                    /* [heads * 128][E] */
 	const void *const *attn_k, *const *attn_v;    /* [kv_heads * 128][E] */
-	const void *const *attn_o;                    /* [E][heads * 128] */
+	const void *const *attn_o;                    /* [E][heads * 128]; in Q8_0 / Q4_0, heads * 128 = 256, 512 .. 4096 */
 	const float *const *q_norm, *const *k_norm;   /* OLMoE [E]; NULL otherwise */
 	const float *const *ffn_norm;                 /* [E] */
 	const float *const *gate_inp;                 /* router [NE][E] */
